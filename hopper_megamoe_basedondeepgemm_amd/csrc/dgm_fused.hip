@@ -168,24 +168,31 @@ DGM_DEV v4i hi4(v8i v) { return __builtin_shufflevector(v, v, 4, 5, 6, 7); }
 constexpr int FT = 512;        // threads per workgroup (8 waves)
 constexpr int NW = FT / 64;
 
-template <int KT1, int KT2, int ACT>
+template <int KT1, int KT2, int ACT, bool BIG>
 struct FusedSmem {
   // U4 per lane per K-tile: E2M1 (32 codes), E4M3 / int8 (two 16-byte halves), NVFP4 as f16
   // (four ops of eight halves)
   static constexpr int BV = ACT == DGM_ACT_MXFP4 ? 1 : ACT == DGM_ACT_NVFP4 ? 4 : 2;
   static constexpr int KTM = KT1 > KT2 ? KT1 : KT2;
-  int exp_of_route[FUSED_MAX_ROUTES];
-  float route_w[FUSED_MAX_ROUTES];     // routing weight of each route
-  int routes[FUSED_MAX_ROUTES];
-  int prow[FUSED_MAX_ROUTES];          // per pool row: its route's row in `partials` (slot * part_rows + token)
-  static constexpr int PT = ACT == DGM_ACT_NVFP4 ? 1 : FUSED_MAX_ROUTES;
+  static constexpr int MR = BIG ? 1 : FUSED_MAX_ROUTES, BR = BIG ? FUSED_BIG_ROUTES : 1;
+  int exp_of_route[MR];
+  float route_w[MR];                   // routing weight of each route
+  int routes[MR];
+  int prow[MR];                        // per pool row: its route's row in `partials` (slot * part_rows + token)
+  static constexpr int PT = ACT == DGM_ACT_NVFP4 ? 1 : MR;
   int ptok[PT];                        // per pool row: its token (not NVFP4)
-  float pw[PT];                        // per pool row: its routing weight (not NVFP4)
-  int ytok[FUSED_MAX_ROUTES];          // per pool row: its token when that token has no other local
+  float pw[BIG ? BR : PT];             // per pool row: its routing weight (not NVFP4)
+  int ytok[MR];                        // per pool row: its token when that token has no other local
                                        // route (the L2 unit writes y itself), else -1
+  // BIG: the same tables for up to FUSED_BIG_ROUTES routes, packed. prt, per pool row: its token
+  // (bits 0-11), its slot (bits 12-15) and whether the token has no other local route (bit 31);
+  // expb: each route's local expert or -1; nslotb: each token's local routes
+  uint32_t prt[BR];
+  int16_t expb[BR];
+  uint8_t nslotb[BR];
   int act[FUSED_MAX_LOCAL];
   int aoff[FUSED_MAX_LOCAL + 1];
-  int nslot[FUSED_MAX_TOKENS];
+  int nslot[BIG ? 1 : FUSED_MAX_TOKENS];
   int wsum[NW][2];
   int meta[4];
   uint32_t amask[FUSED_MAX_LOCAL / 32];   // (early streaming) active local experts, bit e
@@ -193,6 +200,7 @@ struct FusedSmem {
     struct {                           // dispatch only
       int cnt[FUSED_MAX_LOCAL];
       int eoff[FUSED_MAX_LOCAL];
+      int wcnt[BIG ? NW : 1][BIG ? FUSED_MAX_LOCAL : 1];   // (BIG) routes per wave and expert
     };
     U4 bst[KTM][64][BV];               // B slab in matrix-core fragment order
   };
@@ -309,8 +317,8 @@ DGM_DEV void route_key_ranks(S& s, int R, int lane, int wv, int* part) {
   for (int j = 0; j < QW; ++j) rk += (uint32_t)__builtin_amdgcn_readlane((int)key, QW * wv + j) < key ? 1 : 0;
   part[wv * 64 + lane] = rk;
 }
-// r / d for 0 <= r < 1024 and 1 <= d <= 16 as a multiply and a shift: with m = ceil(2^20 / d),
-// r m / 2^20 exceeds r / d by less than 2^-10 < 1 / d, so the floors agree (also checked for
+// r / d for 0 <= r < 4096 and 1 <= d <= 16 as a multiply and a shift: with m = ceil(2^20 / d),
+// r m / 2^20 exceeds r / d by less than 2^-8 < 1 / d, so the floors agree (also checked for
 // every such r and d). A route's token is route / top-k; the generic integer division it
 // replaces is a long dependent sequence (M=16 and NVFP4 layer calls: 0.2-1.4 us faster).
 DGM_DEV uint32_t div_magic(int d) { return (0x100000u + (uint32_t)d - 1u) / (uint32_t)d; }
@@ -347,6 +355,95 @@ DGM_DEV void wave_dispatch(S& s, int R, uint32_t tkm, int lane, const int* part)
   }
   // per active expert: count = next offset - offset (the wave's LDS stores above come first)
   for (int i = lane; i < base; i += 64) s.cnt[s.act[i]] = s.aoff[i + 1] - s.aoff[i];
+}
+
+// The pool table of R <= FUSED_BIG_ROUTES routes (any expert distribution): a stable counting
+// sort. Wave w owns the routes w RW .. +RW - 1 in order, 64 per step. Within a step a route's rank
+// among its expert's routes is the count of lower lanes with the same expert (their mask from one
+// ballot per expert-id bit); the wave's running count per expert gives the steps before. An
+// exclusive sum over the waves per expert, then over experts, places every route: the canonical
+// pool order without a sort of each segment (an expert's whole segment may be one expert's 4096
+// routes) and without an order that depends on atomics. Every workgroup does this for itself: the
+// table is ready 6.5 us after kernel entry at 4096 routes (the split path's k_dispatch, one
+// workgroup that ranks each route against all earlier ones, takes 177 us there, 54 us at 2056).
+template <class S>
+DGM_DEV void big_dispatch(S& s, const int64_t* __restrict__ topk_idx, const float* __restrict__ topk_w, int R, int M,
+                          int topk, uint32_t tkm, int expert_begin, int E_local) {
+  constexpr int STEPS = FUSED_BIG_ROUTES / (NW * 64);
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int RW = ((R + NW * 64 - 1) / (NW * 64)) * 64;         // routes per wave
+  int64_t g[STEPS];
+  float w[STEPS];
+#pragma unroll
+  for (int k = 0; k < STEPS; ++k) {                             // (all requested before any is used)
+    const int r = wv * RW + 64 * k + lane;
+    const bool have = 64 * k < RW && r < R;
+    g[k] = -1;
+    w[k] = 0.f;
+    if (have) {
+      g[k] = topk_idx[r];
+      w[k] = topk_w[r];
+    }
+  }
+  for (int i = tid; i < NW * FUSED_MAX_LOCAL; i += FT) (&s.wcnt[0][0])[i] = 0;
+  __syncthreads();
+  int e[STEPS], pos[STEPS];
+#pragma unroll
+  for (int k = 0; k < STEPS; ++k) {
+    e[k] = -1;
+    pos[k] = 0;
+    if (64 * k < RW) {                                          // (uniform)
+      const int r = wv * RW + 64 * k + lane;
+      const int64_t l = g[k] - expert_begin;
+      const bool mine = r < R && g[k] >= 0 && l >= 0 && l < E_local;
+      const int ee = mine ? (int)l : 0;
+      e[k] = mine ? ee : -1;
+      if (r < R) s.expb[r] = (int16_t)e[k];
+      uint64_t peers = __ballot(mine);
+#pragma unroll
+      for (int b = 0; (1 << b) < FUSED_MAX_LOCAL; ++b) {
+        const uint64_t m = __ballot((ee >> b) & 1);
+        peers &= (ee >> b) & 1 ? m : ~m;
+      }
+      const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(peers >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)peers, 0u));
+      const int before = s.wcnt[wv][ee];
+      pos[k] = before + rank;
+      // (every lane has read its count before the first lane of each expert moves it on; the next
+      // step reads it back: one wave's LDS operations complete in order)
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      if (mine && rank == 0) s.wcnt[wv][ee] = before + (int)__popcll(peers);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+  }
+  __syncthreads();
+  for (int x = tid; x < E_local; x += FT) {
+    int base = 0;
+#pragma unroll
+    for (int v = 0; v < NW; ++v) {
+      const int c = s.wcnt[v][x];
+      s.wcnt[v][x] = base;
+      base += c;
+    }
+    s.cnt[x] = base;
+  }
+  for (int t = tid; t < M; t += FT) {
+    int n = 0;
+    for (int sl = 0; sl < topk; ++sl) n += s.expb[t * topk + sl] >= 0 ? 1 : 0;
+    s.nslotb[t] = (uint8_t)n;
+  }
+  __syncthreads();
+  scan_experts(s, E_local);
+#pragma unroll
+  for (int k = 0; k < STEPS; ++k) {
+    if (64 * k < RW && e[k] >= 0) {
+      const int r = wv * RW + 64 * k + lane;
+      const int q = s.eoff[e[k]] + s.wcnt[wv][e[k]] + pos[k];
+      const int t = div_small(r, tkm);
+      s.prt[q] = (uint32_t)t | ((uint32_t)(r - t * topk) << 12) | (s.nslotb[t] == 1 ? 1u << 31 : 0u);
+      s.pw[q] = w[k];
+    }
+  }
+  __syncthreads();
 }
 
 // A bounded wait expired: the error counter is set (it stays set until the caller clears it),
@@ -702,11 +799,18 @@ DGM_DEV long long wall_clock() { return (long long)__builtin_amdgcn_s_memrealtim
 // The kernel's forms (one instantiation each; the launch picks one): plain, FEIN, and the
 // opt-in EARLY and TAIL (A-MXFP at H = 3072, small routed sets: the last round of L1 units as
 // half units).
-constexpr int FORM_PLAIN = 0, FORM_FEIN = 1, FORM_EARLY = 2, FORM_TAIL = 3;
+// BIG: up to FUSED_BIG_ROUTES routes and tokens (A-MXFP, FP8F128), with packed tables (the plain
+// form's would not fit the LDS beside the slab), the counting-sort dispatch, and combine counters
+// packed on their lines (with many tokens their updates spread over enough lines).
+// Such calls ran as the split path's launches (dispatch, k_l1, k_l2, combine), whose L1 and L2 do
+// not stream: 512 tokens of E384 H3072 I1280, A-MXFP8, whole call 1227 -> 497 us, one of eight
+// ranks' experts, A-MXFP4, 367 -> 135 us.
+constexpr int FORM_PLAIN = 0, FORM_FEIN = 1, FORM_EARLY = 2, FORM_TAIL = 3, FORM_BIG = 4;
 template <int KT1, int KT2, int ACT, int FORM>
 __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
-  constexpr bool FEIN = FORM == FORM_FEIN, EARLY = FORM == FORM_EARLY, TAIL = FORM == FORM_TAIL;
-  using Smem = FusedSmem<KT1, KT2, ACT>;
+  constexpr bool FEIN = FORM == FORM_FEIN, EARLY = FORM == FORM_EARLY, TAIL = FORM == FORM_TAIL, BIG = FORM == FORM_BIG;
+  using Smem = FusedSmem<KT1, KT2, ACT, BIG>;
+  constexpr int CSTRIDE = BIG ? 1 : CNT_LINE;               // ints per combine counter
   __shared__ Smem s;
   constexpr int FB = ACT == DGM_ACT_MXFP4 ? 4 : 0;        // B operand format
   constexpr int KH = KT1 / 2;                               // L1 K-tiles per wave (K halves)
@@ -741,7 +845,7 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
   int parity = 0;
   int* cset = nullptr;
   int* l1_done = nullptr;      // expert slot a: l1_done[a * CNT_LINE]
-  int* comb = nullptr;         // pair i: comb[i * CNT_LINE]
+  int* comb = nullptr;         // pair i: comb[i * CSTRIDE]
   auto take_parity = [&]() __attribute__((always_inline)) {
     asm volatile("" : "+v"(parity_v));    // (the wait for the load is placed here)
     parity = __builtin_amdgcn_readfirstlane(parity_v) & 1;
@@ -855,9 +959,13 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
   SlabRegs<KT1, ACT, FEIN, false> pre;     // an L1 slab on its way to LDS
 
   // ---------------------------------------------------------------- dispatch (every WG)
-  for (int t = tid; t < p.M; t += FT) s.nslot[t] = 0;
+  if constexpr (!BIG) {
+    for (int t = tid; t < p.M; t += FT) s.nslot[t] = 0;
+  }
   if (EARLY && tid < FUSED_MAX_LOCAL / 32) s.amask[tid] = 0u;
-  if (p.select) {
+  if constexpr (BIG) {
+    big_dispatch(s, p.topk_idx, p.topk_w, R, p.M, p.topk, tkm, p.expert_begin, p.E_local);
+  } else if (p.select) {
     // top-k from the frontend's keys, as the frontend would have done: the keys of TC tokens at
     // a time go through LDS (the slab area, unused until the L1 phase; one coalesced pass),
     // then one wave selects per token
@@ -920,7 +1028,9 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
       s.route_w[r] = p.topk_w[r];
     }
   }
-  for (int e = tid; e < p.E_local; e += FT) s.cnt[e] = 0;   // (shares LDS with the key staging)
+  if constexpr (!BIG) {
+    for (int e = tid; e < p.E_local; e += FT) s.cnt[e] = 0;   // (shares LDS with the key staging)
+  }
   if constexpr (!FEIN) take_parity();      // (the routing loads above have returned)
   if constexpr (!EARLY && !FEIN) count_start();
   if constexpr (ACT == DGM_ACT_NVFP4) {
@@ -956,7 +1066,9 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
     }
     count_start();
   }
-  if (R <= 64) {
+  if constexpr (BIG) {
+    // (the table is built)
+  } else if (R <= 64) {
     // key ranks counted by every wave, then one wave sorts the routes (the other waves wait
     // at the barrier); the parts are staged in the L1 epilogue's up-sum buffer (unused until
     // then)
@@ -992,6 +1104,7 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
     __syncthreads();
   }
   const int n_active = s.meta[0];
+  if constexpr (!BIG) {
   for (int q = tid; q < s.meta[1]; q += FT) {
     const int r = s.routes[q], t = div_small(r, tkm);
     s.prow[q] = (r - t * p.topk) * p.part_rows + t;
@@ -1002,6 +1115,29 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
     // (NVFP4: always through the combine; its kernel has no registers to spare for the y store)
     s.ytok[q] = ACT != DGM_ACT_NVFP4 && s.nslot[t] == 1 ? t : -1;
   }
+  }
+  // The table's views: a pool row's token, row in `partials` and token when it is the token's only
+  // local route (else -1); a token's local routes
+  auto tok_of = [](int q) __attribute__((always_inline)) {
+    if constexpr (BIG) return (int)(s.prt[q] & 0xfffu);
+    else return s.ptok[q];
+  };
+  auto prow_of = [part_rows = p.part_rows](int q) __attribute__((always_inline)) {
+    if constexpr (BIG) {
+      const uint32_t v = s.prt[q];
+      return (int)((v >> 12) & 15u) * part_rows + (int)(v & 0xfffu);
+    } else {
+      return s.prow[q];
+    }
+  };
+  auto ytok_of = [](int q) __attribute__((always_inline)) {
+    if constexpr (BIG) return (s.prt[q] >> 31) ? (int)(s.prt[q] & 0xfffu) : -1;
+    else return s.ytok[q];
+  };
+  auto nslot_of = [](int t) __attribute__((always_inline)) {
+    if constexpr (BIG) return (int)s.nslotb[t];
+    else return s.nslot[t];
+  };
   if (st && tid == 0) st[1] = wall_clock();
   if (blockIdx.x == 0) {
     int* meta = (int*)p.pool_out;
@@ -1025,11 +1161,23 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
       goff[a] = s.aoff[a];
       if (a < n_active) gact[a] = s.act[a];
     }
-    for (int r = tid; r < s.meta[1]; r += FT) grt[r] = s.routes[r];
+    for (int r = tid; r < s.meta[1]; r += FT) {
+      if constexpr (BIG) grt[r] = (int)(s.prt[r] & 0xfffu) * p.topk + (int)((s.prt[r] >> 12) & 15u);
+      else grt[r] = s.routes[r];
+    }
     // tokens without a local route: y row = 0
-    for (int i = tid; i < p.M * (H / 8); i += FT) {
-      int t = i / (H / 8);
-      if (s.nslot[t] == 0) reinterpret_cast<U4*>(p.y + (size_t)t * H)[i % (H / 8)] = U4{0, 0, 0, 0};
+    if constexpr (!BIG) {
+      for (int i = tid; i < p.M * (H / 8); i += FT) {
+        int t = i / (H / 8);
+        if (s.nslot[t] == 0) reinterpret_cast<U4*>(p.y + (size_t)t * H)[i % (H / 8)] = U4{0, 0, 0, 0};
+      }
+    }
+  }
+  if constexpr (BIG) {      // (spread over the grid: one workgroup's pass over every row takes 16 us)
+    if (p.phases & 2) {
+      for (int t = (int)blockIdx.x; t < p.M; t += (int)gridDim.x)
+        if (s.nslotb[t] == 0)
+          for (int i = tid; i < H / 8; i += FT) reinterpret_cast<U4*>(p.y + (size_t)t * H)[i] = U4{0, 0, 0, 0};
     }
   }
   // The other counter set, cleared one line per thread, spread over the grid (its last user,
@@ -1129,7 +1277,7 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
     // LDS read each, where route -> token / top-k and route -> weight were a dependent read and
     // an integer division on the first slab's path (0.5-1.7 us per layer call). NVFP4 keeps the
     // route-table reads: with the tables its kernel spills more registers.
-    auto load_slab = [xv, xs, tkm](SlabRegs<KT1, ACT, FEIN, false>& r, int a, int s0) __attribute__((always_inline)) {
+    auto load_slab = [xv, xs, tkm, tok_of](SlabRegs<KT1, ACT, FEIN, false>& r, int a, int s0) __attribute__((always_inline)) {
       if constexpr (ACT == DGM_ACT_NVFP4) {
         const int* rts = s.routes + s.aoff[a] + s0;
         slab_load<KT1, ACT, FEIN, false>(r, xv, xs, XB, s.aoff[a + 1] - s.aoff[a] - s0,
@@ -1138,7 +1286,7 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
       } else {
         const int q0r = s.aoff[a] + s0;
         slab_load<KT1, ACT, FEIN, false>(r, xv, xs, XB, s.aoff[a + 1] - q0r,
-                                         [q0r](int cc) { return s.ptok[q0r + cc]; },
+                                         [q0r, tok_of](int cc) { return tok_of(q0r + cc); },
                                          [q0r](int cc) { return s.pw[q0r + cc]; });
       }
     };
@@ -1635,7 +1783,7 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
                                 [](int) { return 0.f; });
     };
     // arrivals of item (unit v, slab s0): its routes' outputs for the unit's blocks are complete
-    auto arrive = [comb, tid, tkm](int v, int s0) __attribute__((always_inline)) {
+    auto arrive = [comb, tid, tkm, tok_of, ytok_of](int v, int s0) __attribute__((always_inline)) {
       // (the top-k multiplier and the thread index made opaque: what derives from them is
       // computed here, not kept live across the work loop, where it would cost registers or a
       // spill)
@@ -1647,9 +1795,9 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
       // (the route's token from the pool-row table: the division by top-k it replaces sat between
       // the item's two barriers and cost 0.4-1.8 us per layer call; NVFP4 has no table)
       for (int i = i0; i < 16 * RB && i / RB < n; i += FT)
-        if (ACT == DGM_ACT_NVFP4 || s.ytok[r0 + i / RB] < 0) {   // (a token's only local route writes y itself)
-          const int t = ACT == DGM_ACT_NVFP4 ? div_small(s.routes[r0 + i / RB], tk) : s.ptok[r0 + i / RB];
-          __hip_atomic_fetch_add(&comb[(t * NBL2 + RB * b + i % RB) * CNT_LINE], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (ACT == DGM_ACT_NVFP4 || ytok_of(r0 + i / RB) < 0) {   // (a token's only local route writes y itself)
+          const int t = ACT == DGM_ACT_NVFP4 ? div_small(s.routes[r0 + i / RB], tk) : tok_of(r0 + i / RB);
+          __hip_atomic_fetch_add(&comb[(t * NBL2 + RB * b + i % RB) * CSTRIDE], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     };
     // units v0 and G + v0 first, then claims (offset by 2 G)
@@ -1902,14 +2050,14 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
       wait_vm_le<ACT == DGM_ACT_NVFP4 ? 2 * KT2 : KT2>();
       if (s0 + c < n) {
         // each route's output rounded to bf16 (the reference's per-route rule), stored slot-major
-        uint16_t* dst = p.partials + (size_t)s.prow[r0 + s0 + c] * H + (NW * RB * b + RB * wv) * 16 + 4 * kq;
+        uint16_t* dst = p.partials + (size_t)prow_of(r0 + s0 + c) * H + (NW * RB * b + RB * wv) * 16 + 4 * kq;
 #pragma unroll
         for (int j = 0; j < RB; ++j)
           st_agent64(dst + 16 * j, (uint64_t)f32_to_bf16(acc[j][0]) | ((uint64_t)f32_to_bf16(acc[j][1]) << 16) |
                                        ((uint64_t)f32_to_bf16(acc[j][2]) << 32) | ((uint64_t)f32_to_bf16(acc[j][3]) << 48));
         // a token with no other local route: its y rows are this route's output (the combine of
         // one bf16 route output), written here; no arrival, no combine
-        const int yt = ACT == DGM_ACT_NVFP4 ? -1 : s.ytok[r0 + s0 + c];
+        const int yt = ACT == DGM_ACT_NVFP4 ? -1 : ytok_of(r0 + s0 + c);
         if (yt >= 0) {
           uint16_t* yd = p.y + (size_t)yt * H + (NW * RB * b + RB * wv) * 16 + 4 * kq;
 #pragma unroll
@@ -1972,20 +2120,23 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
     const int P = p.M * NBL2;
     for (int i = (int)blockIdx.x + wv * (int)gridDim.x; i < P; i += (int)gridDim.x * NW) {
       {
-        const int need = s.nslot[i / NBL2];
-        if (need > DIRECT_Y && lane == 0) spin_until2(&comb[i * CNT_LINE], need, p.spin_limit, err, p.host_err);
+        const int need = nslot_of(i / NBL2);
+        if (need > DIRECT_Y && lane == 0) spin_until2(&comb[i * CSTRIDE], need, p.spin_limit, err, p.host_err);
         __atomic_signal_fence(__ATOMIC_SEQ_CST);    // (the partial loads below come after the wait)
         const int t = i / NBL2, row = (i % NBL2) * BR + 2 * lane;
         // (y rows of tokens without a local route: zeroed by workgroup 0; with one: written by its
         // L2 unit, except NVFP4's)
-        if (s.nslot[t] > DIRECT_Y) {
+        if (need > DIRECT_Y) {
           // every local route's two values are requested first (one round trip for all of
           // them), then summed in slot order (fp32; a route of another rank adds nothing)
           constexpr int MAXK = 16;                       // (topk <= 16, checked on the host)
           const int tk = p.topk;
           int ex[MAXK];                                  // (all read before any is tested)
 #pragma unroll
-          for (int sl = 0; sl < MAXK; ++sl) ex[sl] = s.exp_of_route[min(t * tk + sl, FUSED_MAX_ROUTES - 1)];
+          for (int sl = 0; sl < MAXK; ++sl) {
+            if constexpr (BIG) ex[sl] = s.expb[min(t * tk + sl, FUSED_BIG_ROUTES - 1)];
+            else ex[sl] = s.exp_of_route[min(t * tk + sl, FUSED_MAX_ROUTES - 1)];
+          }
           uint32_t v[MAXK], use = 0;
 #pragma unroll
           for (int sl = 0; sl < MAXK; ++sl) {
@@ -2026,11 +2177,11 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
   if (st && tid == 0) st[5] = wall_clock();
 }
 
-// per device, per (shape slot, format, form: plain / FEIN / EARLY / TAIL): the resident grid; per
+// per device, per (shape slot, format, form: plain / FEIN / EARLY / TAIL / BIG): the resident grid; per
 // (shape slot, format): the last launch's grid and form (the grid is what the device keeps
 // resident at once, so it depends on the device's CU count)
 constexpr int GRID_DEVICES = 64;
-struct GridCache { int blocks[3][5][4] = {}; int last[3][5] = {}; int form[3][5] = {}; };
+struct GridCache { int blocks[3][5][5] = {}; int last[3][5] = {}; int form[3][5] = {}; };
 GridCache g_grid[GRID_DEVICES];
 
 GridCache& grid_cache() {
@@ -2092,8 +2243,16 @@ bool use_tail(const FusedParams& prm) {
   return !prm.fe_in && (prm.phases & 1) && (long long)prm.M * prm.topk <= 32 && (prm.debug & 16);
 }
 
+// The large-batch form where the plain form's tables end (1024 routes, 256 tokens).
+bool use_big(const FusedParams& prm) {
+  return !prm.fe_in && !prm.select && ((long long)prm.M * prm.topk > FUSED_MAX_ROUTES || prm.M > FUSED_MAX_TOKENS);
+}
+
 template <int KT1, int KT2, int ACT>
 int launch_fused_fe(const FusedParams& prm, int slot, hipStream_t stream, bool coop) {
+  if constexpr (ACT == DGM_ACT_MXFP4 || ACT == DGM_ACT_MXFP8 || ACT == DGM_ACT_FP8F128) {
+    if (use_big(prm)) return launch_fused_t<KT1, KT2, ACT, FORM_BIG>(prm, slot, stream, coop);
+  }
   if constexpr (ACT == DGM_ACT_MXFP4 || ACT == DGM_ACT_MXFP8) {
     if (use_early(prm, ACT)) return launch_fused_t<KT1, KT2, ACT, FORM_EARLY>(prm, slot, stream, coop);
     if constexpr (KT1 == 24) {

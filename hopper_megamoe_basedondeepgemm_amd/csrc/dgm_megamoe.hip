@@ -893,10 +893,13 @@ int dgm_check_fused_args(const DgmMoeArgs* A) {
   return 0;
 }
 
-// The persistent kernel's limits (route, token, expert and combine-block counts of its LDS tables)
+// The persistent kernel's limits (route, token, expert and combine-block counts of its LDS tables):
+// QoQ and NVFP4 the plain form's, the other formats the large-batch form's (unless the kernel runs
+// the frontend itself)
 static bool fused_fits(const DgmMoeArgs* A) {
-  return A->num_tokens * A->topk <= FUSED_MAX_ROUTES && A->num_local_experts <= FUSED_MAX_LOCAL &&
-         A->num_tokens <= FUSED_MAX_TOKENS && A->hidden / 64 <= FUSED_MAX_NB64;
+  const bool big = A->act_format != DGM_ACT_QOQ && A->act_format != DGM_ACT_NVFP4 && !A->fe_in_mega;
+  return A->num_tokens * A->topk <= (big ? FUSED_BIG_ROUTES : FUSED_MAX_ROUTES) && A->num_local_experts <= FUSED_MAX_LOCAL &&
+         A->num_tokens <= (big ? FUSED_BIG_ROUTES : FUSED_MAX_TOKENS) && A->hidden / 64 <= FUSED_MAX_NB64;
 }
 
 // One launch of the persistent kernel running `phases` (FusedParams::phases) of the layer, with

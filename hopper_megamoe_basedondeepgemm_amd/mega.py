@@ -733,12 +733,14 @@ def fused_workgroups(b):
     return _lib.load().dgm_fused_workgroups(b.hidden, b.intermediate_hidden, b.act_code)
 
 
-FUSED_FORMS = {0: "plain", 1: "in-kernel frontend", 2: "early weight streaming", 3: "tail half units"}
+FUSED_FORMS = {0: "plain", 1: "in-kernel frontend", 2: "early weight streaming", 3: "tail half units",
+               4: "large batch"}
 
 
 def fused_last_form(b):
     """The form the persistent kernel's last launch for this buffer's shape and format ran (a
-    key of ``FUSED_FORMS``; -1 before the first). Two opt-in forms, both measured slower than the
+    key of ``FUSED_FORMS``; -1 before the first). "large batch" runs beyond 1024 routes or 256 tokens
+    (MXFP4 / MXFP8 / FP8F128 activations). Two opt-in forms, both measured slower than the
     default: early weight streaming for small routed sets (MXFP4 / MXFP8 activations, at most 32
     local routes expected), turned on by the buffer's ``_debug_flags`` bit 3, and tail half units
     for up to 32 routes (A-MXFP4 / A-MXFP8 at H = 3072: the last round of L1 units, when at most
