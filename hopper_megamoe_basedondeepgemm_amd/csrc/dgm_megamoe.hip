@@ -68,6 +68,11 @@ __host__ __device__ inline Pool pool_view(uint8_t* base, int E_local) {
 // its barrier cost 1.1-1.7 us more than the hidden-row reads they save).
 constexpr int FE_ROUTER_TILE = 8;         // tokens per router workgroup in the tiled form
 constexpr int FE_TILE_MIN_TOKENS = 64;
+// Matrix-core router tiles (router_tile_mm) from 112 tokens (seven 16-token tiles) on: 128 tokens
+// 12.6 us against 20.0, 100 tokens 12.8 against 17.9, 64 tokens 12.4 against 13.0, 48 tokens 12.4
+// against 12.8, 32 tokens 12.4 against 10.0 (with the selection launch). Between 48 and 111 tokens
+// the eight-token rows stay: fable_frontend_router_ctas publishes their workgroup counts.
+constexpr int FE_MM_MIN_TOKENS = 112;
 // Phase stamps (the reference's DG_FE_STAMPS, deep_gemm/mega/__init__.py:743-756): with stamps
 // non-null, workgroup b = blockIdx.y * gridDim.x + blockIdx.x < stamp_rows writes row b of 8
 // int64: [0] entry, [3] (router rows) keys and logits stored by all four waves, [5] (cast rows)
@@ -132,6 +137,45 @@ __global__ void __launch_bounds__(256) k_frontend(const uint16_t* __restrict__ x
     if (tid == 0) {
       const long long t = fe_clock();
       st[0] = t_entry; st[1] = 0; st[2] = 0; st[3] = 0; st[4] = 0; st[5] = t;
+      st[6] = fe_hw_position(); st[7] = fe_clock();
+    }
+  }
+}
+
+// The frontend from FE_MM_MIN_TOKENS tokens on: workgroups [0, nr) are router tiles of 16 tokens x
+// 16 experts on the matrix cores (router_tile_mm, experts fastest: with E % 128 == 0 an XCD then
+// keeps one share of the router weights in its L2), the rest cast.
+template <int J>
+__global__ void __launch_bounds__(512, 4) k_frontend_mm(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
+                                                      int M, int E, int act_format, float* __restrict__ logits,
+                                                      uint32_t* __restrict__ keys, int zero_unrouted,
+                                                      uint8_t* __restrict__ q, uint8_t* __restrict__ sf, int nr,
+                                                      long long* __restrict__ stamps, int stamp_rows) {
+  constexpr int H = J * 512;
+  __shared__ RouterMmSmem sm;
+  const int tid = threadIdx.x, bid = (int)blockIdx.x;
+  long long* st = stamps != nullptr && bid < stamp_rows ? stamps + (size_t)bid * 8 : nullptr;
+  const long long t_entry = st ? fe_clock() : 0;
+  if (bid < nr) {
+    const int ne = (E + 15) / 16;
+    router_tile_mm<J>(x, w, M, E, (bid % ne) * 16, (bid / ne) * 16, logits, keys, zero_unrouted != 0, sm);
+  } else {
+    const int64_t lane0 = (int64_t)(bid - nr) * 512 + tid, nl = (int64_t)((int)gridDim.x - nr) * 512;
+    if (act_format == DGM_ACT_QOQ) {
+      for (int t = (int)(lane0 >> 6); t < M; t += (int)(nl >> 6)) cast_qoq_token<J, false>(x, t, tid & 63, q, sf);
+    } else if (act_format == DGM_ACT_NVFP4) {
+      for (int64_t i = lane0; i < (int64_t)M * (H / 16) * 4; i += nl) cast_lane_nvfp4<false>(x, i, q, sf);
+    } else if (act_format == DGM_ACT_FP8F128) {
+      for (int64_t i = lane0; i < (int64_t)M * (H / 128) * 32; i += nl) cast_lane_fp8f128<false>(x, i, q, sf);
+    } else {
+      for (int64_t i = lane0; i < (int64_t)M * (H / 32) * 8; i += nl) cast_lane_mx<false>(x, act_format, i, q, sf);
+    }
+  }
+  if (st) {
+    __syncthreads();
+    if (tid == 0) {
+      const long long t = fe_clock();
+      st[0] = t_entry; st[1] = 0; st[2] = 0; st[3] = bid < nr ? t : 0; st[4] = 0; st[5] = bid < nr ? 0 : t;
       st[6] = fe_hw_position(); st[7] = fe_clock();
     }
   }
@@ -711,6 +755,8 @@ extern "C" {
 
 }  // extern "C"
 
+static bool fe_mm(int num_tokens, bool router) { return router && num_tokens >= FE_MM_MIN_TOKENS; }
+
 // The frontend launch's grid: router rows (4 experts x 4 tokens per workgroup, 8 tokens from
 // FE_TILE_MIN_TOKENS on) and, beside them, cast rows of one cast lane per thread (QoQ: one wave
 // per token).
@@ -721,6 +767,9 @@ static dim3 fe_grid(int num_tokens, int hidden, int num_experts, int act_format,
                                : act_format == DGM_ACT_FP8F128 ? (int64_t)num_tokens * (hidden / 128) * 32
                                                                : (int64_t)num_tokens * (hidden / 32) * 8;
   const int64_t cast_rows = (flags & DGM_FE_NO_CAST) ? 0 : (cast_threads + (int64_t)rx * 256 - 1) / ((int64_t)rx * 256);
+  if (fe_mm(num_tokens, router))
+    return dim3(((num_experts + 15) / 16) * ((num_tokens + 15) / 16) +
+                ((flags & DGM_FE_NO_CAST) ? 0 : (int)((cast_threads + 511) / 512)));
   const int rtok = num_tokens >= FE_TILE_MIN_TOKENS ? FE_ROUTER_TILE : 4;
   return dim3(rx, (router ? (num_tokens + rtok - 1) / rtok : 0) + (int)cast_rows);
 }
@@ -764,7 +813,7 @@ int dgm_router_topk_launch_stamped(const void* hidden_bf16, const void* router_w
   uint8_t* buf = (uint8_t*)buffer;
   const int J = hidden / 512;
   const int router = router_weight_bf16 ? 1 : 0;
-  const bool tiled = num_tokens >= FE_TILE_MIN_TOKENS;
+  const bool tiled = num_tokens >= FE_TILE_MIN_TOKENS, mm = fe_mm(num_tokens, router != 0);
   const dim3 rg = fe_grid(num_tokens, hidden, num_experts, act_format, flags, router != 0);
   long long* stamp_ptr = (long long*)stamps;
   const uint16_t* x = (const uint16_t*)hidden_bf16;
@@ -773,7 +822,11 @@ int dgm_router_topk_launch_stamped(const void* hidden_bf16, const void* router_w
   uint32_t* keys = (uint32_t*)(buf + L->fe_keys);
   const int zero_unrouted = (flags & DGM_FE_ZERO_ROW_UNROUTED) ? 1 : 0;
 #define DGM_FE(JJ)                                                                                           \
-  if (tiled)                                                                                                 \
+  if (mm)                                                                                                    \
+    hipLaunchKernelGGL((k_frontend_mm<JJ>), rg, dim3(512), 0, stream, x, w, num_tokens, num_experts, act_format, \
+                       logits, keys, zero_unrouted, buf + L->x, buf + L->x_sf,                               \
+                       ((num_experts + 15) / 16) * ((num_tokens + 15) / 16), stamp_ptr, stamp_rows);         \
+  else if (tiled)                                                                                            \
     hipLaunchKernelGGL((k_frontend<JJ, FE_ROUTER_TILE>), rg, dim3(256), 0, stream, x, w, num_tokens, num_experts, \
                        act_format, logits, keys, zero_unrouted, buf + L->x, buf + L->x_sf, router, stamp_ptr, \
                        stamp_rows);                                                                          \
