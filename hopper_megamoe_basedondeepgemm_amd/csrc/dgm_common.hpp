@@ -243,17 +243,6 @@ DGM_DEV v4f mfma_scale_16x16x128_sel(v8i a, v8i b, v4f c, int sa, int sb) {
   return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, FMT_A, FMT_B, OPA, sa, OPB, sb);
 }
 
-// Keeps the scale registers of a chain of block-scaled matrix-core ops allocated until the chain's
-// last op has issued (the result `acc` is an input here), so that no instruction inside the chain
-// writes a register a later op of the chain reads as its scale. With the scale operands taken
-// from loaded dwords (never computed by VALU ops between the ops), the chain's scales are written
-// only by memory loads.
-template <int N>
-DGM_DEV void keep_scales_until(const uint32_t (&r)[N], v4f acc) {
-#pragma unroll
-  for (int i = 0; i < N; ++i) asm volatile("" ::"v"(acc[0]), "v"(r[i]));
-}
-
 // D(16x16 i32) += A(16x64 int8) * B(64x16 int8), exact. Lane l supplies A row l%16 / B column
 // l%16 with 16 K values (lane group l/16 of both operands pairs byte for byte); result
 // register i of lane l is D[4*(l/16) + i][l%16]. (Pinned by the probe test.)

@@ -69,6 +69,17 @@ DGM_DEV void st_agent64(void* p, uint64_t v) {
   __hip_atomic_store((uint64_t*)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 DGM_DEV void st_agent8(uint8_t* p, uint8_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// LATER: read by a later launch only, so an ordinary store, which merges in the L2, does
+template <bool LATER>
+DGM_DEV void st_handoff64(void* p, uint64_t v) {
+  if constexpr (LATER) *reinterpret_cast<uint64_t*>(p) = v;
+  else st_agent64(p, v);
+}
+template <bool LATER>
+DGM_DEV void st_handoff8(uint8_t* p, uint8_t v) {
+  if constexpr (LATER) *p = v;
+  else st_agent8(p, v);
+}
 DGM_DEV uint64_t ld_agent64(const void* p) {
   return __hip_atomic_load((const uint64_t*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -184,23 +195,21 @@ struct FusedSmem {
   float pw[BIG ? BR : PT];             // per pool row: its routing weight (not NVFP4)
   int ytok[MR];                        // per pool row: its token when that token has no other local
                                        // route (the L2 unit writes y itself), else -1
-  // BIG: the same tables for up to FUSED_BIG_ROUTES routes, packed. prt, per pool row: its token
-  // (bits 0-11), its slot (bits 12-15) and whether the token has no other local route (bit 31);
-  // expb: each route's local expert or -1; nslotb: each token's local routes
+  // BIG: the tables of up to FUSED_BIG_ROUTES routes: pw and, per pool row, its token (bits 0-11)
+  // and slot (bits 12-15)
   uint32_t prt[BR];
-  int16_t expb[BR];
-  uint8_t nslotb[BR];
-  int act[FUSED_MAX_LOCAL];
-  int aoff[FUSED_MAX_LOCAL + 1];
-  int nslot[BIG ? 1 : FUSED_MAX_TOKENS];
+  static constexpr int ML = BIG ? FUSED_BIG_LOCAL : FUSED_MAX_LOCAL;
+  int act[ML];
+  int aoff[ML + 1];
+  int nslot[MR == 1 ? 1 : FUSED_MAX_TOKENS];
   int wsum[NW][2];
   int meta[4];
   uint32_t amask[FUSED_MAX_LOCAL / 32];   // (early streaming) active local experts, bit e
   union {
     struct {                           // dispatch only
-      int cnt[FUSED_MAX_LOCAL];
-      int eoff[FUSED_MAX_LOCAL];
-      int wcnt[BIG ? NW : 1][BIG ? FUSED_MAX_LOCAL : 1];   // (BIG) routes per wave and expert
+      int cnt[ML];
+      int eoff[ML];
+      int wcnt[BIG ? NW : 1][BIG ? ML : 1];   // (BIG) routes per wave and expert
     };
     U4 bst[KTM][64][BV];               // B slab in matrix-core fragment order
   };
@@ -227,10 +236,10 @@ struct FusedSmem {
   int claimv[3];            // [0] the claim ahead, [1] prefetch decision, [2] L2: a complete expert
 };
 
-// Exclusive scan of (count, active flag) over n <= FUSED_MAX_LOCAL experts.
+// Exclusive scan of (count, active flag) over n <= S::ML experts.
 template <class S>
 DGM_DEV void scan_experts(S& s, int n) {
-  constexpr int PER = (FUSED_MAX_LOCAL + FT - 1) / FT;
+  constexpr int PER = (S::ML + FT - 1) / FT;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   int c[PER], a[PER], sc = 0, sa = 0;
 #pragma unroll
@@ -364,11 +373,11 @@ DGM_DEV void wave_dispatch(S& s, int R, uint32_t tkm, int lane, const int* part)
 // exclusive sum over the waves per expert, then over experts, places every route: the canonical
 // pool order without a sort of each segment (an expert's whole segment may be one expert's 4096
 // routes) and without an order that depends on atomics. Every workgroup does this for itself: the
-// table is ready 6.5 us after kernel entry at 4096 routes (the split path's k_dispatch, one
-// workgroup that ranks each route against all earlier ones, takes 177 us there, 54 us at 2056).
+// table is ready 6.5 us after kernel entry at 4096 routes (a launch of one workgroup that ranks each
+// route against all earlier ones took 177 us there, 54 us at 2056).
 template <class S>
-DGM_DEV void big_dispatch(S& s, const int64_t* __restrict__ topk_idx, const float* __restrict__ topk_w, int R, int M,
-                          int topk, uint32_t tkm, int expert_begin, int E_local) {
+DGM_DEV void big_dispatch(S& s, const int64_t* __restrict__ topk_idx, const float* __restrict__ topk_w, int R, int topk,
+                          uint32_t tkm, int expert_begin, int E_local) {
   constexpr int STEPS = FUSED_BIG_ROUTES / (NW * 64);
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int RW = ((R + NW * 64 - 1) / (NW * 64)) * 64;         // routes per wave
@@ -385,7 +394,7 @@ DGM_DEV void big_dispatch(S& s, const int64_t* __restrict__ topk_idx, const floa
       w[k] = topk_w[r];
     }
   }
-  for (int i = tid; i < NW * FUSED_MAX_LOCAL; i += FT) (&s.wcnt[0][0])[i] = 0;
+  for (int i = tid; i < NW * S::ML; i += FT) (&s.wcnt[0][0])[i] = 0;
   __syncthreads();
   int e[STEPS], pos[STEPS];
 #pragma unroll
@@ -398,10 +407,9 @@ DGM_DEV void big_dispatch(S& s, const int64_t* __restrict__ topk_idx, const floa
       const bool mine = r < R && g[k] >= 0 && l >= 0 && l < E_local;
       const int ee = mine ? (int)l : 0;
       e[k] = mine ? ee : -1;
-      if (r < R) s.expb[r] = (int16_t)e[k];
       uint64_t peers = __ballot(mine);
 #pragma unroll
-      for (int b = 0; (1 << b) < FUSED_MAX_LOCAL; ++b) {
+      for (int b = 0; (1 << b) < S::ML; ++b) {
         const uint64_t m = __ballot((ee >> b) & 1);
         peers &= (ee >> b) & 1 ? m : ~m;
       }
@@ -426,11 +434,6 @@ DGM_DEV void big_dispatch(S& s, const int64_t* __restrict__ topk_idx, const floa
     }
     s.cnt[x] = base;
   }
-  for (int t = tid; t < M; t += FT) {
-    int n = 0;
-    for (int sl = 0; sl < topk; ++sl) n += s.expb[t * topk + sl] >= 0 ? 1 : 0;
-    s.nslotb[t] = (uint8_t)n;
-  }
   __syncthreads();
   scan_experts(s, E_local);
 #pragma unroll
@@ -439,9 +442,48 @@ DGM_DEV void big_dispatch(S& s, const int64_t* __restrict__ topk_idx, const floa
       const int r = wv * RW + 64 * k + lane;
       const int q = s.eoff[e[k]] + s.wcnt[wv][e[k]] + pos[k];
       const int t = div_small(r, tkm);
-      s.prt[q] = (uint32_t)t | ((uint32_t)(r - t * topk) << 12) | (s.nslotb[t] == 1 ? 1u << 31 : 0u);
+      s.prt[q] = (uint32_t)t | ((uint32_t)(r - t * topk) << 12);
       s.pw[q] = w[k];
     }
+  }
+  __syncthreads();
+}
+
+// (BIG, the L2 launch) the pool table from the one the L1 launch published, in one round trip:
+// every entry that could be in use is requested before the counts are known.
+template <class S>
+DGM_DEV void big_table_load(S& s, const uint8_t* __restrict__ pool, int R, int topk, uint32_t tkm, int E_local) {
+  constexpr int STEPS = FUSED_BIG_ROUTES / FT, EST = S::ML / FT;
+  const int tid = threadIdx.x;
+  const int* meta = reinterpret_cast<const int*>(pool);
+  const int* act = reinterpret_cast<const int*>(pool + 256 + a256i(E_local * 4));
+  const int* off = reinterpret_cast<const int*>(pool + 256 + 2 * a256i(E_local * 4));
+  const int* rts = reinterpret_cast<const int*>(pool + 256 + 2 * a256i(E_local * 4) + a256i((E_local + 1) * 4));
+  int r[STEPS], a[EST], o[EST];
+  const int m0 = meta[0], m1 = meta[1];
+#pragma unroll
+  for (int k = 0; k < EST; ++k) {
+    a[k] = act[min(tid + k * FT, E_local - 1)];
+    o[k] = off[min(tid + k * FT, E_local - 1)];
+  }
+#pragma unroll
+  for (int k = 0; k < STEPS; ++k) r[k] = rts[min(tid + k * FT, R - 1)];
+#pragma unroll
+  for (int k = 0; k < EST; ++k)
+    if (tid + k * FT < m0) {
+      s.act[tid + k * FT] = a[k];
+      s.aoff[tid + k * FT] = o[k];
+    }
+#pragma unroll
+  for (int k = 0; k < STEPS; ++k)
+    if (tid + k * FT < m1) {
+      const int t = div_small(r[k], tkm);
+      s.prt[tid + k * FT] = (uint32_t)t | ((uint32_t)(r[k] - t * topk) << 12);
+    }
+  if (tid == 0) {
+    s.meta[0] = m0;
+    s.meta[1] = m1;
+    s.aoff[m0] = m1;
   }
   __syncthreads();
 }
@@ -799,18 +841,22 @@ DGM_DEV long long wall_clock() { return (long long)__builtin_amdgcn_s_memrealtim
 // The kernel's forms (one instantiation each; the launch picks one): plain, FEIN, and the
 // opt-in EARLY and TAIL (A-MXFP at H = 3072, small routed sets: the last round of L1 units as
 // half units).
-// BIG: up to FUSED_BIG_ROUTES routes and tokens (A-MXFP, FP8F128), with packed tables (the plain
-// form's would not fit the LDS beside the slab), the counting-sort dispatch, and combine counters
-// packed on their lines (with many tokens their updates spread over enough lines).
-// Such calls ran as the split path's launches (dispatch, k_l1, k_l2, combine), whose L1 and L2 do
-// not stream: 512 tokens of E384 H3072 I1280, A-MXFP8, whole call 1227 -> 497 us, one of eight
-// ranks' experts, A-MXFP4, 367 -> 135 us.
+// BIG: up to FUSED_BIG_ROUTES routes and tokens and FUSED_BIG_LOCAL local experts (A-MXFP, FP8F128),
+// with packed tables (the plain form's would not fit the LDS beside the slab) and the counting-sort
+// dispatch. It runs one phase per launch (L1, or L2 without the combine, which is a launch of its
+// own) and so has no wait on another workgroup: calls beyond the plain form's limits never needed
+// the whole grid resident, and two of them on two streams must not wait for each other's CUs.
+// E384 H3072 I1280, 512 tokens, whole call: A-MXFP8 456 us (259 L1, 151 L2; 1.71 + 0.89 GB read,
+// 6.6 and 5.9 TB/s), one of eight ranks' experts, A-MXFP4, 106 us. The kernels it replaced (a
+// one-workgroup dispatch, L1 and L2 that load an item's weights before its first op) took 1227 and
+// 367 us with the VALU router. Bound by the weight stream and, in L2, the items' fixed cost.
+// Measured and not taken: the whole layer in one launch (455 / 101 us, but with the waits), runs of
+// consecutive units per claim, whose slab is staged once (+4 %: the runs' uneven end).
 constexpr int FORM_PLAIN = 0, FORM_FEIN = 1, FORM_EARLY = 2, FORM_TAIL = 3, FORM_BIG = 4;
 template <int KT1, int KT2, int ACT, int FORM>
 __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
   constexpr bool FEIN = FORM == FORM_FEIN, EARLY = FORM == FORM_EARLY, TAIL = FORM == FORM_TAIL, BIG = FORM == FORM_BIG;
   using Smem = FusedSmem<KT1, KT2, ACT, BIG>;
-  constexpr int CSTRIDE = BIG ? 1 : CNT_LINE;               // ints per combine counter
   __shared__ Smem s;
   constexpr int FB = ACT == DGM_ACT_MXFP4 ? 4 : 0;        // B operand format
   constexpr int KH = KT1 / 2;                               // L1 K-tiles per wave (K halves)
@@ -845,7 +891,7 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
   int parity = 0;
   int* cset = nullptr;
   int* l1_done = nullptr;      // expert slot a: l1_done[a * CNT_LINE]
-  int* comb = nullptr;         // pair i: comb[i * CSTRIDE]
+  int* comb = nullptr;         // pair i: comb[i * CNT_LINE]
   auto take_parity = [&]() __attribute__((always_inline)) {
     asm volatile("" : "+v"(parity_v));    // (the wait for the load is placed here)
     parity = __builtin_amdgcn_readfirstlane(parity_v) & 1;
@@ -924,7 +970,7 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
   // L1 epilogue and the phase change instead of after it.
   constexpr int KR1 = KT1 % 12 == 0 ? 12 : KT1;
   constexpr int RING = KR1 > KT2 ? KR1 : KT2;
-  constexpr bool HANDOFF = KR1 >= KT2;
+  constexpr bool HANDOFF = KR1 >= KT2 && !BIG;
   U4 wr[RING];
   uint32_t sr[ACT == DGM_ACT_NVFP4 ? RING : 1];
   // The L1 phase's wave w streams 16-row block pair pp = w & 3 (16 of a unit's 64 features),
@@ -964,7 +1010,8 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
   }
   if (EARLY && tid < FUSED_MAX_LOCAL / 32) s.amask[tid] = 0u;
   if constexpr (BIG) {
-    big_dispatch(s, p.topk_idx, p.topk_w, R, p.M, p.topk, tkm, p.expert_begin, p.E_local);
+    if (p.phases & 1) big_dispatch(s, p.topk_idx, p.topk_w, R, p.topk, tkm, p.expert_begin, p.E_local);
+    else big_table_load(s, p.pool_out, R, p.topk, tkm, p.E_local);
   } else if (p.select) {
     // top-k from the frontend's keys, as the frontend would have done: the keys of TC tokens at
     // a time go through LDS (the slab area, unused until the L1 phase; one coalesced pass),
@@ -1116,8 +1163,7 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
     s.ytok[q] = ACT != DGM_ACT_NVFP4 && s.nslot[t] == 1 ? t : -1;
   }
   }
-  // The table's views: a pool row's token, row in `partials` and token when it is the token's only
-  // local route (else -1); a token's local routes
+  // The table's views: a pool row's token and its row in `partials`
   auto tok_of = [](int q) __attribute__((always_inline)) {
     if constexpr (BIG) return (int)(s.prt[q] & 0xfffu);
     else return s.ptok[q];
@@ -1130,16 +1176,8 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
       return s.prow[q];
     }
   };
-  auto ytok_of = [](int q) __attribute__((always_inline)) {
-    if constexpr (BIG) return (s.prt[q] >> 31) ? (int)(s.prt[q] & 0xfffu) : -1;
-    else return s.ytok[q];
-  };
-  auto nslot_of = [](int t) __attribute__((always_inline)) {
-    if constexpr (BIG) return (int)s.nslotb[t];
-    else return s.nslot[t];
-  };
   if (st && tid == 0) st[1] = wall_clock();
-  if (blockIdx.x == 0) {
+  if (blockIdx.x == 0 && (!BIG || (p.phases & 1))) {
     int* meta = (int*)p.pool_out;
     int* gcnt = (int*)(p.pool_out + 256);
     int* gact = (int*)(p.pool_out + 256 + a256i(p.E_local * 4));
@@ -1171,13 +1209,6 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
         int t = i / (H / 8);
         if (s.nslot[t] == 0) reinterpret_cast<U4*>(p.y + (size_t)t * H)[i % (H / 8)] = U4{0, 0, 0, 0};
       }
-    }
-  }
-  if constexpr (BIG) {      // (spread over the grid: one workgroup's pass over every row takes 16 us)
-    if (p.phases & 2) {
-      for (int t = (int)blockIdx.x; t < p.M; t += (int)gridDim.x)
-        if (s.nslotb[t] == 0)
-          for (int i = tid; i < H / 8; i += FT) reinterpret_cast<U4*>(p.y + (size_t)t * H)[i] = U4{0, 0, 0, 0};
     }
   }
   // The other counter set, cleared one line per thread, spread over the grid (its last user,
@@ -1579,7 +1610,7 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
       const bool bcast = last_slab && q1 < UI;
       if (tid == 0 && bcast) s.claimv[0] = more ? ahead : -1;
       __syncthreads();                                   // (1) up sums visible, slab free
-      if (tid == 0 && pend >= 0) __hip_atomic_fetch_add(&l1_done[pend * CNT_LINE], pend_w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (!BIG && tid == 0 && pend >= 0) __hip_atomic_fetch_add(&l1_done[pend * CNT_LINE], pend_w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       pend = -1;
       int q2 = UI;
       if (bcast) {
@@ -1678,8 +1709,8 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
                                ((uint64_t)(__shfl(w, c + 32) & 0xffffu) << 32) |
                                ((uint64_t)(__shfl(w, c + 48) & 0xffffu) << 48);
           if (valid && lane < 16) {
-            st_agent64(p.mid + (size_t)row * MB + 8 * pr, w64);
-            if ((ip & 1) == 0) st_agent8(p.mid_sf + (size_t)row * (I / 32) + (pr >> 1), (uint8_t)code);
+            st_handoff64<BIG>(p.mid + (size_t)row * MB + 8 * pr, w64);
+            if ((ip & 1) == 0) st_handoff8<BIG>(p.mid_sf + (size_t)row * (I / 32) + (pr >> 1), (uint8_t)code);
           }
         } else {
           // E4M3 with a power-of-two scale per 32 (MXFP8: 2^ceil(log2(max(amax, 1e-30) / 448)))
@@ -1695,8 +1726,8 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
           const int src_lo = lane < 16 ? c : c + 32, src_hi = lane < 16 ? c + 16 : c + 48;
           const uint64_t w64 = (uint64_t)__shfl(w, src_lo) | ((uint64_t)__shfl(w, src_hi) << 32);
           if (valid && lane < 32) {
-            st_agent64(p.mid + (size_t)row * MB + 16 * pr + (lane < 16 ? 0 : 8), w64);
-            if ((ip & 1) == 0 && lane < 16) st_agent8(p.mid_sf + (size_t)row * (I / 32) + (pr >> 1), (uint8_t)code);
+            st_handoff64<BIG>(p.mid + (size_t)row * MB + 16 * pr + (lane < 16 ? 0 : 8), w64);
+            if ((ip & 1) == 0 && lane < 16) st_handoff8<BIG>(p.mid_sf + (size_t)row * (I / 32) + (pr >> 1), (uint8_t)code);
           }
         }
       }
@@ -1721,7 +1752,7 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
     } else {
       wait_mem();             // the last item's stores (and the dummy ring reads)
       __syncthreads();
-      if (tid == 0 && pend >= 0) __hip_atomic_fetch_add(&l1_done[pend * CNT_LINE], pend_w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (!BIG && tid == 0 && pend >= 0) __hip_atomic_fetch_add(&l1_done[pend * CNT_LINE], pend_w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
   if (st && tid == 0) st[2] = wall_clock();
@@ -1777,13 +1808,14 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
     };
     const uint8_t* midv = p.mid;
     const uint8_t* mids = p.mid_sf;
-    auto load_slab = [midv, mids](SlabRegs<KT2, ACT2, true>& r, int a, int s0) __attribute__((always_inline)) {
+    // (BIG: the rows are an earlier launch's, read through the cache)
+    auto load_slab = [midv, mids](SlabRegs<KT2, ACT2, !BIG, true>& r, int a, int s0) __attribute__((always_inline)) {
       const int rb = s.aoff[a] + s0;
-      slab_load<KT2, ACT2, true, true>(r, midv, mids, MB, s.aoff[a + 1] - rb, [rb](int cc) { return rb + cc; },
+      slab_load<KT2, ACT2, !BIG, true>(r, midv, mids, MB, s.aoff[a + 1] - rb, [rb](int cc) { return rb + cc; },
                                 [](int) { return 0.f; });
     };
     // arrivals of item (unit v, slab s0): its routes' outputs for the unit's blocks are complete
-    auto arrive = [comb, tid, tkm, tok_of, ytok_of](int v, int s0) __attribute__((always_inline)) {
+    auto arrive = [comb, tid, tkm, tok_of](int v, int s0) __attribute__((always_inline)) {
       // (the top-k multiplier and the thread index made opaque: what derives from them is
       // computed here, not kept live across the work loop, where it would cost registers or a
       // spill)
@@ -1795,9 +1827,9 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
       // (the route's token from the pool-row table: the division by top-k it replaces sat between
       // the item's two barriers and cost 0.4-1.8 us per layer call; NVFP4 has no table)
       for (int i = i0; i < 16 * RB && i / RB < n; i += FT)
-        if (ACT == DGM_ACT_NVFP4 || ytok_of(r0 + i / RB) < 0) {   // (a token's only local route writes y itself)
+        if (ACT == DGM_ACT_NVFP4 || s.ytok[r0 + i / RB] < 0) {   // (a token's only local route writes y itself)
           const int t = ACT == DGM_ACT_NVFP4 ? div_small(s.routes[r0 + i / RB], tk) : tok_of(r0 + i / RB);
-          __hip_atomic_fetch_add(&comb[(t * NBL2 + RB * b + i % RB) * CSTRIDE], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_fetch_add(&comb[(t * NBL2 + RB * b + i % RB) * CNT_LINE], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     };
     // units v0 and G + v0 first, then claims (offset by 2 G)
@@ -1812,12 +1844,12 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
     int s0 = 0;
     static_assert(KT2 <= RING, "the L2 ring in the shared tile registers");
     uint32_t sd[SW2], sn[SW2];
-    SlabRegs<KT2, ACT2, true> pre;
+    SlabRegs<KT2, ACT2, !BIG, true> pre;
     int ready = -1;           // (thread 0) an active expert whose L1 arrival is known complete
     bool seen = false;        // (stamps) first L1 arrival observed
     int pv = -1, ps0 = 0;     // the previous item, whose arrivals are not sent yet
     int pr_a = 0, pr_n = 0;
-    if (p.phases & 1) {
+    if (!BIG && (p.phases & 1)) {
       // probes of the L1 arrivals of the first two units' experts, answered while the L1
       // phase's last stores complete
       if (tid == 0 && q0 < U2) {
@@ -1852,7 +1884,7 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
     // at the item's start; its loads complete while the tiles and scales above are in flight).
     // (NVFP4 stages it at the item's start: measured no faster this way.)
     bool pre1 = false;
-    if (ACT != DGM_ACT_NVFP4 && q0 < U2 && (!(p.phases & 1) || __builtin_amdgcn_readfirstlane(s.claimv[1]) != 0)) {
+    if (ACT != DGM_ACT_NVFP4 && q0 < U2 && (BIG || !(p.phases & 1) || __builtin_amdgcn_readfirstlane(s.claimv[1]) != 0)) {
       load_slab(pre, q0 / UPE, 0);
       pre1 = true;
     }
@@ -1868,7 +1900,7 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
       } else if (key != staged) {    // not prefetched: wait for the expert's L1 units, then stage
         const long long w0 = st ? wall_clock() : 0;
         if (a != ready) {
-          if (tid == 0 && (p.phases & 1)) spin_until2(&l1_done[a * CNT_LINE], L1W * QN1, p.spin_limit, err, p.host_err);
+          if (!BIG && tid == 0 && (p.phases & 1)) spin_until2(&l1_done[a * CNT_LINE], L1W * QN1, p.spin_limit, err, p.host_err);
           ready = a;
         }
         __syncthreads();
@@ -1882,7 +1914,7 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
           slab_store(s, pre);
         } else {
           const int rb = r0 + s0;
-          stage_slab<KT2, ACT2, true>(s, p.mid, p.mid_sf, MB, n - s0, [rb](int cc) { return rb + cc; });
+          stage_slab<KT2, ACT2, !BIG>(s, p.mid, p.mid_sf, MB, n - s0, [rb](int cc) { return rb + cc; });
         }
         staged = key;
         __syncthreads();
@@ -1895,11 +1927,15 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
       // prefetch the next item's slab if it differs and its expert's L1 is complete
       bool pf = false;
       if (has_next && nkey != key) {
+        if constexpr (BIG) {
+          pf = true;
+        } else {
         if (tid == 0)
           s.claimv[1] = !(p.phases & 1) || na == ready || na == s.claimv[2] ||
                         __hip_atomic_load(&l1_done[na * CNT_LINE], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= L1W * QN1;
         __syncthreads();
         pf = __builtin_amdgcn_readfirstlane(s.claimv[1]) != 0;
+        }
         if (pf) {
           ready = na;
           load_slab(pre, na, ns0);
@@ -2053,11 +2089,12 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
         uint16_t* dst = p.partials + (size_t)prow_of(r0 + s0 + c) * H + (NW * RB * b + RB * wv) * 16 + 4 * kq;
 #pragma unroll
         for (int j = 0; j < RB; ++j)
-          st_agent64(dst + 16 * j, (uint64_t)f32_to_bf16(acc[j][0]) | ((uint64_t)f32_to_bf16(acc[j][1]) << 16) |
+          st_handoff64<BIG>(dst + 16 * j, (uint64_t)f32_to_bf16(acc[j][0]) | ((uint64_t)f32_to_bf16(acc[j][1]) << 16) |
                                        ((uint64_t)f32_to_bf16(acc[j][2]) << 32) | ((uint64_t)f32_to_bf16(acc[j][3]) << 48));
         // a token with no other local route: its y rows are this route's output (the combine of
         // one bf16 route output), written here; no arrival, no combine
-        const int yt = ACT == DGM_ACT_NVFP4 ? -1 : ytok_of(r0 + s0 + c);
+        int yt = -1;
+        if constexpr (ACT != DGM_ACT_NVFP4 && !BIG) yt = WIDE && (p.phases & 4) ? -1 : s.ytok[r0 + s0 + c];
         if (yt >= 0) {
           uint16_t* yd = p.y + (size_t)yt * H + (NW * RB * b + RB * wv) * 16 + 4 * kq;
 #pragma unroll
@@ -2070,7 +2107,7 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
       const bool bcast = last_slab && q1 < U2;
       if (tid == 0 && bcast) s.claimv[0] = more ? ahead : -1;
       __syncthreads();                                   // (1) previous outputs complete, slab free
-      if (pv >= 0) arrive(pv, ps0);
+      if (!BIG && pv >= 0 && !(WIDE && (p.phases & 4))) arrive(pv, ps0);
       pv = q0;
       ps0 = s0;
       int q2 = U2;
@@ -2098,7 +2135,7 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
     }
     wait_mem();               // the last item's outputs (and the dummy reads)
     __syncthreads();
-    if (pv >= 0) arrive(pv, ps0);
+    if (!BIG && pv >= 0 && !(WIDE && (p.phases & 4))) arrive(pv, ps0);
   };
   if (p.phases & 2) {
     if (halves) l2_phase(std::integral_constant<int, 1>{});
@@ -2113,15 +2150,15 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
   // -> bf16 y. No wave waits for another's pair (measured: 1-1.5 us less at M=2-4 than eight
   // consecutive pairs per workgroup behind one barrier). The waits are only on L2 items, which
   // never wait on this phase.
-  if (p.phases & 2) {
+  if (!BIG && (p.phases & (WIDE ? 6 : 2)) == 2) {
     constexpr int DIRECT_Y = ACT == DGM_ACT_NVFP4 ? 0 : 1;   // routes per token that need no combine
     constexpr int BR = 16 * NW;
     static_assert(BR == 2 * 64, "a wave's lanes cover a block, two rows each");
     const int P = p.M * NBL2;
     for (int i = (int)blockIdx.x + wv * (int)gridDim.x; i < P; i += (int)gridDim.x * NW) {
       {
-        const int need = nslot_of(i / NBL2);
-        if (need > DIRECT_Y && lane == 0) spin_until2(&comb[i * CSTRIDE], need, p.spin_limit, err, p.host_err);
+        const int need = s.nslot[i / NBL2];
+        if (need > DIRECT_Y && lane == 0) spin_until2(&comb[i * CNT_LINE], need, p.spin_limit, err, p.host_err);
         __atomic_signal_fence(__ATOMIC_SEQ_CST);    // (the partial loads below come after the wait)
         const int t = i / NBL2, row = (i % NBL2) * BR + 2 * lane;
         // (y rows of tokens without a local route: zeroed by workgroup 0; with one: written by its
@@ -2133,10 +2170,7 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
           const int tk = p.topk;
           int ex[MAXK];                                  // (all read before any is tested)
 #pragma unroll
-          for (int sl = 0; sl < MAXK; ++sl) {
-            if constexpr (BIG) ex[sl] = s.expb[min(t * tk + sl, FUSED_BIG_ROUTES - 1)];
-            else ex[sl] = s.exp_of_route[min(t * tk + sl, FUSED_MAX_ROUTES - 1)];
-          }
+          for (int sl = 0; sl < MAXK; ++sl) ex[sl] = s.exp_of_route[min(t * tk + sl, FUSED_MAX_ROUTES - 1)];
           uint32_t v[MAXK], use = 0;
 #pragma unroll
           for (int sl = 0; sl < MAXK; ++sl) {
@@ -2243,9 +2277,9 @@ bool use_tail(const FusedParams& prm) {
   return !prm.fe_in && (prm.phases & 1) && (long long)prm.M * prm.topk <= 32 && (prm.debug & 16);
 }
 
-// The large-batch form where the plain form's tables end (1024 routes, 256 tokens).
+// The large-batch form where the plain form's tables end (1024 routes, 256 tokens, 512 local experts).
 bool use_big(const FusedParams& prm) {
-  return !prm.fe_in && !prm.select && ((long long)prm.M * prm.topk > FUSED_MAX_ROUTES || prm.M > FUSED_MAX_TOKENS);
+  return (long long)prm.M * prm.topk > FUSED_MAX_ROUTES || prm.M > FUSED_MAX_TOKENS || prm.E_local > FUSED_MAX_LOCAL;
 }
 
 template <int KT1, int KT2, int ACT>

@@ -7,10 +7,9 @@ constexpr int FUSED_MAX_ROUTES = 1024;   // tokens * topk per call
 constexpr int FUSED_MAX_LOCAL = 512;     // local experts
 constexpr int FUSED_MAX_TOKENS = 256;    // tokens per call
 constexpr int FUSED_MAX_NB64 = 64;       // hidden / 64 (hidden <= 4096); combine uses hidden / 128
-// The large-batch form (A-MXFP4 / A-MXFP8 / FP8F128): routes and tokens per call. Its combine
-// counters are packed (one int each) in the region the plain form's 256 tokens fill with one line
-// each.
+// The large-batch form (A-MXFP4 / A-MXFP8 / FP8F128): routes and tokens per call, local experts.
 constexpr int FUSED_BIG_ROUTES = 4096;
+constexpr int FUSED_BIG_LOCAL = 1024;
 
 // int32 counters in the buffer's counter region. Counters that many workgroups update at once
 // sit on 64-byte lines of their own (device-scope atomics on one line serialize).
@@ -37,8 +36,6 @@ constexpr int CNT_GRID = CNT_TOTAL;
 constexpr int GRID_SLOTS = 32, GRID_STRIDE = 16;
 constexpr int CNT_SET = CNT_GRID + 1024;                 // ints per set
 constexpr int CNT_ALL = CNT_SET0 + 2 * CNT_SET;
-
-static_assert(FUSED_BIG_ROUTES <= FUSED_MAX_TOKENS * CNT_LINE, "packed combine counters fit the region");
 
 inline __host__ __device__ int a256i(int x) { return (x + 255) & ~255; }
 
@@ -81,7 +78,8 @@ struct FusedParams {
   int16_t fast_math;
   // Phases run by this launch: bit 0 dispatch + L1 (intermediate rows to `mid`, recv stats),
   // bit 1 L2 + combine. 3 = the whole layer; 1 then 2 = the split API's two launches (the
-  // second reads the top-k written by the first and does not wait for L1 arrivals).
+  // second reads the top-k written by the first and does not wait for L1 arrivals). Bit 2 (with
+  // bit 1): no combine: the route outputs only, no arrival and no wait on another workgroup.
   int16_t phases;
   int16_t debug;            // bit 0: one bounded wait that expires (tests of the error reporting);
                             // bit 1 (QoQ): the int32 L1 accumulators to `stamps` [routes][2 I];

@@ -1,5 +1,6 @@
-// MegaMoE layer kernels for MI355X (gfx950): router/top-k frontend, dispatch, L1 and L2
-// grouped block-scaled GEMMs on the matrix cores, and the top-k combine.
+// MegaMoE layer on MI355X (gfx950): the frontend kernels (router, top-k, activation casts), the
+// combine of the calls that run the layer as several launches, and the C ABI. The experts run on
+// the persistent kernel (dgm_fused.hip).
 //
 // Data layout in HBM (one GPU's share of the EP layer):
 //  * weights: matrix-core fragment order written by dgm_transform_fp4_weights. A 16-row x
@@ -11,11 +12,7 @@
 //    per-expert pool is the list of routes; no row copies).
 //  * intermediate (L1 -> L2): [pool row, I/2 | I] codes + [pool row, I/32] scales, pool rows
 //    in (expert asc, token asc, slot asc) order.
-//  * route outputs: fp32 [token * topk + slot, H]; the combine sums valid slots in slot order.
-//
-// Matrix-core use: swap-AB. The weight tile is the 16-row A operand, up to 16 routed tokens
-// form the narrow B operand (one 16-token slab), V_MFMA_SCALE_F32_16X16X128_F8F6F4 applies
-// the E8M0 block scales of both operands in hardware (no dequantisation on the VALU).
+//  * route outputs: bf16 [topk][tokens][H]; the combine sums valid slots in slot order.
 #include "dgm_common.hpp"
 #include "dgm_abi_internal.hpp"
 #include "dgm_fused.hpp"
@@ -24,35 +21,6 @@
 using namespace dgm;
 
 namespace {
-
-struct alignas(16) U4 { uint32_t x, y, z, w; };
-
-DGM_DEV v8i u4_to_v8i(U4 a) { v8i r = {(int)a.x, (int)a.y, (int)a.z, (int)a.w, 0, 0, 0, 0}; return r; }
-DGM_DEV v8i u8_to_v8i(U4 a, U4 b) {
-  v8i r = {(int)a.x, (int)a.y, (int)a.z, (int)a.w, (int)b.x, (int)b.y, (int)b.z, (int)b.w};
-  return r;
-}
-
-// ------------------------------------------------------------------ pool table
-struct Pool {
-  int* meta;      // [0] n_active, [1] total routes
-  int* counts;    // [E_local]
-  int* active;    // [n_active] local expert ids, ascending
-  int* offsets;   // [n_active + 1] first pool row of each active expert
-  int* routes;    // [total] route id (token * topk + slot) of each pool row
-};
-
-__host__ __device__ inline size_t a256(size_t x) { return (x + 255) & ~(size_t)255; }
-
-__host__ __device__ inline Pool pool_view(uint8_t* base, int E_local) {
-  Pool p;
-  p.meta = (int*)base;
-  p.counts = (int*)(base + 256);
-  p.active = (int*)(base + 256 + a256((size_t)E_local * 4));
-  p.offsets = (int*)(base + 256 + 2 * a256((size_t)E_local * 4));
-  p.routes = (int*)(base + 256 + 2 * a256((size_t)E_local * 4) + a256((size_t)(E_local + 1) * 4));
-  return p;
-}
 
 // ------------------------------------------------------------------ frontend
 // Router rows of the grid (by < ceil(M / RTOK)): workgroup (bx, by) computes the logits and
@@ -214,358 +182,6 @@ __global__ void __launch_bounds__(256) k_keys_bf16(const uint16_t* __restrict__ 
   keys[i] = topk_key(bf16_to_f32(logits[i]), (int)(i % E));
 }
 
-// ------------------------------------------------------------------ dispatch
-// One workgroup: per-expert counts, canonical pool order (token asc, slot asc) by rank of
-// the route id among the routes of its expert, exclusive scans over experts, stats update.
-constexpr int DISPATCH_THREADS = 1024;
-constexpr int MAX_ROUTES_DISPATCH = 4096;
-constexpr int MAX_LOCAL_EXPERTS = 1024;
-
-__global__ void __launch_bounds__(DISPATCH_THREADS) k_dispatch(const int64_t* __restrict__ topk_idx, int routes_n,
-                                                               int expert_begin, int E_local,
-                                                               uint8_t* __restrict__ pool_base,
-                                                               int* __restrict__ recv_stats) {
-  __shared__ int s_exp[MAX_ROUTES_DISPATCH];
-  __shared__ int s_cnt[MAX_LOCAL_EXPERTS];
-  __shared__ int s_off[MAX_LOCAL_EXPERTS];
-  __shared__ int s_act[MAX_LOCAL_EXPERTS];
-  __shared__ int s_wave[DISPATCH_THREADS / 64][2];
-  Pool P = pool_view(pool_base, E_local);
-  const int tid = threadIdx.x;
-  for (int e = tid; e < E_local; e += DISPATCH_THREADS) s_cnt[e] = 0;
-  for (int r = tid; r < routes_n; r += DISPATCH_THREADS) {
-    int64_t g = topk_idx[r];
-    int64_t l = g - expert_begin;
-    s_exp[r] = (g >= 0 && l >= 0 && l < E_local) ? (int)l : -1;
-  }
-  __syncthreads();
-  for (int r = tid; r < routes_n; r += DISPATCH_THREADS)
-    if (s_exp[r] >= 0) atomicAdd(&s_cnt[s_exp[r]], 1);
-  __syncthreads();
-  // exclusive scans of counts and of the active flags over experts (E_local <= 1024)
-  int c = 0, a = 0;
-  if (tid < E_local) { c = s_cnt[tid]; a = c > 0 ? 1 : 0; }
-  int lane = tid & 63, wv = tid >> 6;
-  int ic = c, ia = a;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    int oc = __shfl_up(ic, off), oa = __shfl_up(ia, off);
-    if (lane >= off) { ic += oc; ia += oa; }
-  }
-  if (lane == 63) { s_wave[wv][0] = ic; s_wave[wv][1] = ia; }
-  __syncthreads();
-  int bc = 0, ba = 0;
-  for (int i = 0; i < wv; ++i) { bc += s_wave[i][0]; ba += s_wave[i][1]; }
-  int exc = bc + ic - c, exa = ba + ia - a;
-  if (tid < E_local) {
-    s_off[tid] = exc;
-    P.counts[tid] = c;
-    if (a) { s_act[exa] = tid; P.active[exa] = tid; P.offsets[exa] = exc; }
-    if (recv_stats) recv_stats[tid] += c;
-  }
-  __syncthreads();
-  if (tid == 0) {
-    int tot = 0, na = 0;
-    for (int i = 0; i < DISPATCH_THREADS / 64; ++i) { tot += s_wave[i][0]; na += s_wave[i][1]; }
-    P.meta[0] = na;
-    P.meta[1] = tot;
-    P.offsets[na] = tot;
-  }
-  for (int r = tid; r < routes_n; r += DISPATCH_THREADS) {
-    int e = s_exp[r];
-    if (e < 0) continue;
-    int rank = 0;
-    for (int q = 0; q < r; ++q) rank += (s_exp[q] == e) ? 1 : 0;
-    P.routes[s_off[e] + rank] = r;
-  }
-}
-
-// ------------------------------------------------------------------ L1: gate/up + SwiGLU + requant
-// Workgroup = NWV waves; item = (active expert a, 16 NWV intermediate features q). Wave w owns
-// the (gate, up) block pair p = NWV q + w (16 features). Both weight tiles of every K-tile are
-// loaded into registers up front (one 1 KB coalesced run per tile), the 16-token B slab is
-// staged once per workgroup in LDS in fragment order, then 2 * KT matrix-core ops run.
-// Epilogue: clamp, silu(g)*u*w, requant of the item's features across its waves.
-// MXFP4 / MXFP8 (2 waves): gate/up rounded to bf16, per-32 E8M0 requant.
-// FP8F128 (4 waves): the activation's fp32 scale of each (token, K-tile) multiplies that
-// K-tile's product (the op runs with a unit activation scale into a zero accumulator, then
-// acc += s * part), fp32 gate/up, per-64 power-of-two FP8 requant stored as two equal per-32
-// E8M0 bytes (so the MXFP8 L2 reads it).
-template <int ACT> constexpr int l1_waves() { return ACT == DGM_ACT_FP8F128 ? 4 : 2; }
-
-template <int KT, int ACT>
-struct L1Smem {
-  static constexpr int BYTES = ACT == DGM_ACT_MXFP4 ? 16 : 32;
-  static constexpr int KG = (KT + 3) / 4;
-  U4 b[KT][64][BYTES / 16];
-  uint32_t bs[KG][64];
-  float bsf[ACT == DGM_ACT_FP8F128 ? KT : 1][16];    // FP8F128: per (K-tile, slab column) scale
-  float amax[l1_waves<ACT>()][16];
-};
-
-template <int KT, int ACT>
-__global__ void __launch_bounds__(64 * l1_waves<ACT>()) k_l1(const uint8_t* __restrict__ w1v,
-                                                           const uint32_t* __restrict__ w1s,
-                                                           const uint8_t* __restrict__ x, const uint8_t* __restrict__ xsf,
-                                                           const float* __restrict__ topk_w, uint8_t* __restrict__ pool_base,
-                                                           int E_local, int I, int topk, float clamp, int fast_math,
-                                                           uint8_t* __restrict__ mid, uint8_t* __restrict__ mid_sf) {
-  constexpr int NWV = l1_waves<ACT>(), NT = 64 * NWV;
-  constexpr bool F128 = ACT == DGM_ACT_FP8F128;
-  constexpr int KG = (KT + 3) / 4;
-  constexpr int XB = ACT == DGM_ACT_MXFP4 ? KT * 64 : KT * 128;   // x row bytes (H/2 or H)
-  constexpr int H = KT * 128;
-  __shared__ L1Smem<KT, ACT> sm;
-  Pool P = pool_view(pool_base, E_local);
-  const int n_active = P.meta[0];
-  const int QN = I / (16 * NWV);
-  const int NB1 = I / 8;            // 16-row blocks of the 2I-row L1 weight
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int midb = ACT == DGM_ACT_MXFP4 ? I / 2 : I;
-  const int items = n_active * QN;
-  for (int item = blockIdx.x; item < items; item += gridDim.x) {
-    const int a = item / QN, q = item % QN;
-    const int e = P.active[a];
-    const int r0 = P.offsets[a], n = P.offsets[a + 1] - r0;
-    const int p = NWV * q + wv;
-    // ---- A operands: gate tile (block 2p) and up tile (block 2p+1) for every K-tile
-    const uint8_t* gbase = w1v + ((size_t)(e * NB1 + 2 * p) * KT) * 1024 + lane * 16;
-    const uint8_t* ubase = gbase + (size_t)KT * 1024;
-    U4 ag[KT], au[KT];
-#pragma unroll
-    for (int kt = 0; kt < KT; ++kt) {
-      ag[kt] = *reinterpret_cast<const U4*>(gbase + kt * 1024);
-      au[kt] = *reinterpret_cast<const U4*>(ubase + kt * 1024);
-    }
-    uint32_t sg[KG], su[KG];
-    const uint32_t* gs = w1s + ((size_t)(e * NB1 + 2 * p) * KG) * 64 + lane;
-#pragma unroll
-    for (int g = 0; g < KG; ++g) { sg[g] = gs[g * 64]; su[g] = gs[(KG + g) * 64]; }
-
-    for (int s0 = 0; s0 < n; s0 += 16) {
-      // ---- stage the B slab (routes s0..s0+15 of this expert) in fragment order
-      __syncthreads();
-      for (int f = threadIdx.x; f < KT * 64; f += NT) {
-        int kt = f >> 6, l = f & 63, c = l & 15;
-        U4 v0 = {0, 0, 0, 0}, v1 = {0, 0, 0, 0};
-        if (s0 + c < n) {
-          int t = P.routes[r0 + s0 + c] / topk;
-          if (ACT == DGM_ACT_MXFP4) {
-            v0 = *reinterpret_cast<const U4*>(x + (size_t)t * XB + kt * 64 + (l >> 4) * 16);
-          } else {
-            // E4M3 operand: lane group g holds K = 16 g .. +16 (bytes 0-15) and
-            // K = 64 + 16 g .. +16 (bytes 16-31) of the 128-wide K-tile.
-            const uint8_t* src = x + (size_t)t * XB + kt * 128 + (l >> 4) * 16;
-            v0 = *reinterpret_cast<const U4*>(src);
-            v1 = *reinterpret_cast<const U4*>(src + 64);
-          }
-        }
-        sm.b[kt][l][0] = v0;
-        if (ACT != DGM_ACT_MXFP4) sm.b[kt][l][ACT != DGM_ACT_MXFP4 ? 1 : 0] = v1;
-      }
-      for (int f = threadIdx.x; f < KG * 64; f += NT) {
-        int g = f >> 6, l = f & 63, c = l & 15;
-        uint32_t w = 0x7f7f7f7fu;
-        if (!F128 && s0 + c < n) {
-          int t = P.routes[r0 + s0 + c] / topk;
-          w = 0;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            int kt = 4 * g + j;
-            uint32_t b = kt < KT ? xsf[(size_t)t * (H / 32) + kt * 4 + (l >> 4)] : 127u;
-            w |= b << (8 * j);
-          }
-        }
-        sm.bs[g][l] = w;
-      }
-      if constexpr (F128) {
-        for (int f = threadIdx.x; f < KT * 16; f += NT) {
-          const int kt = f >> 4, c = f & 15;
-          float v = 0.f;
-          if (s0 + c < n) v = reinterpret_cast<const float*>(xsf)[(size_t)(P.routes[r0 + s0 + c] / topk) * KT + kt];
-          sm.bsf[kt][c] = v;
-        }
-      }
-      __syncthreads();
-      // ---- matrix cores. Scale bytes are selected from the loaded scale dwords by the op's
-      // byte select (no VALU writes to a scale operand inside the chain of matrix-core ops)
-      v4f accg = {0.f, 0.f, 0.f, 0.f}, accu = {0.f, 0.f, 0.f, 0.f};
-      v4f accg1 = {0.f, 0.f, 0.f, 0.f}, accu1 = {0.f, 0.f, 0.f, 0.f};
-      uint32_t bsw[KG];
-#pragma unroll
-      for (int g = 0; g < KG; ++g) bsw[g] = sm.bs[g][lane];
-      const int c = lane & 15;
-      static_for<KT>([&](auto kc) {
-        constexpr int kt = decltype(kc)::value;
-        v8i bop;
-        if (ACT == DGM_ACT_MXFP4) bop = u4_to_v8i(sm.b[kt][lane][0]);
-        else bop = u8_to_v8i(sm.b[kt][lane][0], sm.b[kt][lane][ACT != DGM_ACT_MXFP4 ? 1 : 0]);
-        constexpr int FB = ACT == DGM_ACT_MXFP4 ? 4 : 0;
-        constexpr int SEL = kt & 3;
-        if constexpr (F128) {
-          // this K-tile's products with a unit activation scale, promoted by the token's scale
-          const v4f z = {0.f, 0.f, 0.f, 0.f};
-          const v4f tg = mfma_scale_16x16x128_sel<4, FB, SEL, SEL>(u4_to_v8i(ag[kt]), bop, z, (int)sg[kt >> 2], (int)bsw[kt >> 2]);
-          const v4f tu = mfma_scale_16x16x128_sel<4, FB, SEL, SEL>(u4_to_v8i(au[kt]), bop, z, (int)su[kt >> 2], (int)bsw[kt >> 2]);
-          const float sx = sm.bsf[kt][c];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            accg[i] = fmaf(sx, tg[i], accg[i]);
-            accu[i] = fmaf(sx, tu[i], accu[i]);
-          }
-        } else if constexpr (kt < KT / 2) {
-          accg = mfma_scale_16x16x128_sel<4, FB, SEL, SEL>(u4_to_v8i(ag[kt]), bop, accg, (int)sg[kt >> 2], (int)bsw[kt >> 2]);
-          accu = mfma_scale_16x16x128_sel<4, FB, SEL, SEL>(u4_to_v8i(au[kt]), bop, accu, (int)su[kt >> 2], (int)bsw[kt >> 2]);
-        } else {
-          accg1 = mfma_scale_16x16x128_sel<4, FB, SEL, SEL>(u4_to_v8i(ag[kt]), bop, accg1, (int)sg[kt >> 2], (int)bsw[kt >> 2]);
-          accu1 = mfma_scale_16x16x128_sel<4, FB, SEL, SEL>(u4_to_v8i(au[kt]), bop, accu1, (int)su[kt >> 2], (int)bsw[kt >> 2]);
-        }
-      });
-      if constexpr (F128) {
-        keep_scales_until(sg, accg);
-        keep_scales_until(su, accu);
-        keep_scales_until(bsw, accg);
-        keep_scales_until(bsw, accu);
-      } else {
-        keep_scales_until(sg, accg1);
-        keep_scales_until(su, accu1);
-        keep_scales_until(bsw, accg1);
-        keep_scales_until(bsw, accu1);
-        accg += accg1;
-        accu += accu1;
-      }
-      // ---- epilogue: lane holds features 16p + 4(l/16) + i for slab column c = l % 16
-      const bool valid = s0 + c < n;
-      float act[4];
-      float am = 0.f;
-      float wt = 0.f;
-      if (valid) wt = topk_w[P.routes[r0 + s0 + c]];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float g = fminf(F128 ? accg[i] : round_bf16(accg[i]), clamp);
-        float u = fminf(fmaxf(F128 ? accu[i] : round_bf16(accu[i]), -clamp), clamp);
-        float sg1 = fast_math ? sigmoid<true>(g) : sigmoid<false>(g);
-        act[i] = valid ? ((g * sg1) * u) * wt : 0.f;
-        am = fmaxf(am, fabsf(act[i]));
-      }
-      am = fmaxf(am, __shfl_xor(am, 16));
-      am = fmaxf(am, __shfl_xor(am, 32));
-      if (lane < 16) sm.amax[wv][lane] = am;
-      __syncthreads();
-      am = sm.amax[0][c];
-#pragma unroll
-      for (int w = 1; w < NWV; ++w) am = fmaxf(am, sm.amax[w][c]);
-      if (valid) {
-        const int row = r0 + s0 + c;
-        const int f0 = 16 * p + 4 * (lane >> 4);
-        if (ACT == DGM_ACT_MXFP4) {
-          uint32_t code = ceil_ue8m0_code(fmaxf(am, 1e-30f) / 6.0f);
-          float is = e8m0_inv(code);
-          uint32_t w = 0;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) w |= e2m1_ties_down(act[i] * is) << (4 * i);
-          *reinterpret_cast<uint16_t*>(mid + (size_t)row * midb + f0 / 2) = (uint16_t)w;
-          if (wv == 0 && lane < 16) mid_sf[(size_t)row * (I / 32) + q] = (uint8_t)code;
-        } else {
-          // MXFP8: 2^ceil(log2(max(amax, 1e-30) / 448)); FP8F128: 2^ceil(log2(max(amax / 448,
-          // FLT_MIN)))
-          float ex = F128 ? ceil_log2_f32(fmaxf(am / 448.0f, 1.17549435e-38f))
-                          : ceil_log2_f32(fmaxf(am, 1e-30f) / 448.0f);
-          int code = (int)ex + 127;
-          float is = e8m0_inv((uint32_t)code);
-          uint32_t w = 0;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) w |= e4m3_encode(act[i] * is) << (8 * i);
-          *reinterpret_cast<uint32_t*>(mid + (size_t)row * midb + f0) = w;
-          if (wv == 0 && lane < 16) {
-            if (F128) {
-              mid_sf[(size_t)row * (I / 32) + 2 * q] = (uint8_t)code;
-              mid_sf[(size_t)row * (I / 32) + 2 * q + 1] = (uint8_t)code;
-            } else {
-              mid_sf[(size_t)row * (I / 32) + q] = (uint8_t)code;
-            }
-          }
-        }
-      }
-    }
-  }
-}
-
-// ------------------------------------------------------------------ L2: down projection
-// One wave per item (active expert a, 16 output rows b). A: KT2 tiles in registers; B: the
-// 16-route slab of intermediate rows read straight from L2-resident memory.
-template <int KT, int ACT>
-__global__ void __launch_bounds__(256) k_l2(const uint8_t* __restrict__ w2v, const uint32_t* __restrict__ w2s,
-                                            const uint8_t* __restrict__ mid, const uint8_t* __restrict__ mid_sf,
-                                            uint8_t* __restrict__ pool_base, int E_local, int H, int topk,
-                                            int part_rows, uint16_t* __restrict__ partials) {
-  constexpr int KG = (KT + 3) / 4;
-  constexpr int I = KT * 128;
-  constexpr int MB = ACT == DGM_ACT_MXFP4 ? I / 2 : I;
-  Pool P = pool_view(pool_base, E_local);
-  const int n_active = P.meta[0];
-  const int NB2 = H / 16;
-  const int lane = threadIdx.x & 63;
-  const int items = n_active * NB2;
-  const int waves = gridDim.x * 4;
-  for (int item = blockIdx.x * 4 + (threadIdx.x >> 6); item < items; item += waves) {
-    const int a = item / NB2, b = item % NB2;
-    const int e = P.active[a];
-    const int r0 = P.offsets[a], n = P.offsets[a + 1] - r0;
-    const uint8_t* base = w2v + ((size_t)(e * NB2 + b) * KT) * 1024 + lane * 16;
-    U4 av[KT];
-#pragma unroll
-    for (int kt = 0; kt < KT; ++kt) av[kt] = *reinterpret_cast<const U4*>(base + kt * 1024);
-    uint32_t sa[KG];
-    const uint32_t* sp = w2s + ((size_t)(e * NB2 + b) * KG) * 64 + lane;
-#pragma unroll
-    for (int g = 0; g < KG; ++g) sa[g] = sp[g * 64];
-    const int c = lane & 15, kq = lane >> 4;
-    for (int s0 = 0; s0 < n; s0 += 16) {
-      const bool valid = s0 + c < n;
-      const int row = r0 + s0 + (valid ? c : 0);
-      v4f acc = {0.f, 0.f, 0.f, 0.f};
-      // the activation scale bytes of every K-tile, loaded before the chain of matrix-core ops
-      // into registers of their own (a lane without a route reads its slab's first row: its B
-      // operand is zero, and a real scale byte is finite); the weight scale bytes are selected
-      // from the loaded dwords by the op's byte select, so no VALU op writes a scale operand
-      // inside the chain
-      uint32_t sbv[KT];
-#pragma unroll
-      for (int kt = 0; kt < KT; ++kt) sbv[kt] = mid_sf[(size_t)row * (I / 32) + kt * 4 + kq];
-      static_for<KT>([&](auto kc) {
-        constexpr int kt = decltype(kc)::value;
-        v8i bop;
-        if (ACT == DGM_ACT_MXFP4) {
-          U4 v = {0, 0, 0, 0};
-          if (valid) v = *reinterpret_cast<const U4*>(mid + (size_t)row * MB + kt * 64 + kq * 16);
-          bop = u4_to_v8i(v);
-        } else {
-          U4 v0 = {0, 0, 0, 0}, v1 = {0, 0, 0, 0};
-          if (valid) {
-            const uint8_t* s = mid + (size_t)row * MB + kt * 128 + kq * 16;
-            v0 = *reinterpret_cast<const U4*>(s);
-            v1 = *reinterpret_cast<const U4*>(s + 64);
-          }
-          bop = u8_to_v8i(v0, v1);
-        }
-        constexpr int FB = ACT == DGM_ACT_MXFP4 ? 4 : 0;
-        acc = mfma_scale_16x16x128_sel<4, FB, kt & 3, 0>(u4_to_v8i(av[kt]), bop, acc, (int)sa[kt >> 2], (int)sbv[kt]);
-      });
-      keep_scales_until(sa, acc);
-      keep_scales_until(sbv, acc);
-      if (valid) {
-        // the route's output rounded to bf16, slot-major [topk][part_rows][H]
-        const int rid = P.routes[row];
-        const int t = rid / topk, sl = rid - t * topk;
-        const uint2 o = make_uint2((uint32_t)f32_to_bf16(acc[0]) | ((uint32_t)f32_to_bf16(acc[1]) << 16),
-                                   (uint32_t)f32_to_bf16(acc[2]) | ((uint32_t)f32_to_bf16(acc[3]) << 16));
-        *reinterpret_cast<uint2*>(partials + ((size_t)sl * part_rows + t) * H + b * 16 + 4 * kq) = o;
-      }
-    }
-  }
-}
-
 // ------------------------------------------------------------------ combine
 // y[t, n] = bf16(sum over valid local slots s ascending of float(partials[s, t, n])) (bf16 route
 // outputs, fp32 sum).
@@ -618,25 +234,11 @@ int cu_count() {
   return g_cu_count;
 }
 
-template <int KT1, int KT2, int ACT>
-int launch_experts(const DgmMoeArgs* A, uint8_t* buf, const DgmBufferLayout* L, hipStream_t stream) {
-  const int cus = cu_count();
-  uint8_t* pool = buf + L->pool;
-  int items1 = A->num_local_experts * (A->intermediate / (16 * l1_waves<ACT>()));
-  int grid1 = items1 < cus * 4 ? items1 : cus * 4;
-  hipLaunchKernelGGL((k_l1<KT1, ACT>), dim3(grid1), dim3(64 * l1_waves<ACT>()), 0, stream, (const uint8_t*)A->w1_values,
-                     (const uint32_t*)A->w1_scales, buf + L->x, buf + L->x_sf,
-                     (const float*)(buf + L->topk_weights), pool, A->num_local_experts, A->intermediate,
-                     A->topk, A->activation_clamp, A->fast_math, buf + L->mid, buf + L->mid_sf);
-  int st = dgm_last_launch_status();
-  if (st) return st;
-  int items2 = A->num_local_experts * (A->hidden / 16);
-  int grid2 = (items2 + 3) / 4 < cus * 4 ? (items2 + 3) / 4 : cus * 4;
-  // (FP8F128: the intermediate is FP8 with E8M0 bytes per 32, as MXFP8's)
-  constexpr int ACT2 = ACT == DGM_ACT_FP8F128 ? DGM_ACT_MXFP8 : ACT;
-  hipLaunchKernelGGL((k_l2<KT2, ACT2>), dim3(grid2), dim3(256), 0, stream, (const uint8_t*)A->w2_values,
-                     (const uint32_t*)A->w2_scales, buf + L->mid, buf + L->mid_sf, pool, A->num_local_experts,
-                     A->hidden, A->topk, L->max_tokens, (uint16_t*)(buf + L->partials));
+int launch_combine(const DgmMoeArgs* A, uint8_t* buf, const DgmBufferLayout* L, hipStream_t stream) {
+  dim3 cg((A->hidden / 4 + 255) / 256, A->num_tokens);
+  hipLaunchKernelGGL(k_combine, cg, dim3(256), 0, stream, (const uint16_t*)(buf + L->partials), L->max_tokens,
+                     (const int64_t*)(buf + L->topk_idx), A->num_tokens, A->hidden, A->topk, A->expert_begin,
+                     A->num_local_experts, (uint16_t*)A->y);
   return dgm_last_launch_status();
 }
 
@@ -692,7 +294,7 @@ int dgm_fused_buffer_layout(int max_tokens, int num_experts, int num_local_exper
   DGM_CHECK_ARG(num_local_experts > 0 && num_local_experts <= num_experts, "num_local_experts");
   DGM_CHECK_ARG(hidden % 512 == 0 && intermediate % 128 == 0, "hidden % 512, intermediate % 128");
   DGM_CHECK_ARG(act_format >= DGM_ACT_MXFP4 && act_format <= DGM_ACT_FP8F128, "act_format");
-  DGM_CHECK_ARG((int64_t)max_tokens * topk <= MAX_ROUTES_DISPATCH, "max_tokens * topk <= 4096");
+  DGM_CHECK_ARG((int64_t)max_tokens * topk <= FUSED_BIG_ROUTES, "max_tokens * topk <= 4096");
   // scales: E8M0 bytes per 32 (MXFP); QoQ: fp32 per token repeated over H / 128 slots (the
   // same H / 32 bytes) and fp32 per 64 intermediate features (I / 16 bytes); NVFP4: E4M3
   // bytes per 16; FP8F128: fp32 per 128 K (H / 32 bytes) and E8M0 bytes per 32 intermediate
@@ -926,7 +528,7 @@ int dgm_check_fused_args(const DgmMoeArgs* A) {
                                           A->intermediate, A->act_format);
     if (chk) return chk;
   }
-  DGM_CHECK_ARG(A->num_local_experts > 0 && A->num_local_experts <= MAX_LOCAL_EXPERTS, "num_local_experts");
+  DGM_CHECK_ARG(A->num_local_experts > 0 && A->num_local_experts <= FUSED_BIG_LOCAL, "num_local_experts");
   DGM_CHECK_ARG(A->expert_begin >= 0 && A->expert_begin + A->num_local_experts <= A->num_experts, "expert range");
   DGM_CHECK_ARG(A->act_format >= DGM_ACT_MXFP4 && A->act_format <= DGM_ACT_FP8F128, "act_format");
   DGM_CHECK_ARG(A->act_format != DGM_ACT_QOQ || (A->w1_row_scales && A->w2_row_scales),
@@ -946,15 +548,14 @@ int dgm_check_fused_args(const DgmMoeArgs* A) {
   return 0;
 }
 
-// The persistent kernel's limits (route, token, expert and combine-block counts of its LDS tables):
-// QoQ and NVFP4 the plain form's, the other formats the large-batch form's (unless the kernel runs
-// the frontend itself)
+// The plain persistent form's limits (route, token, expert and combine-block counts of its LDS
+// tables): within them the whole layer is one launch. Beyond them MXFP4, MXFP8 and FP8F128
+// activations run the large-batch form, one launch per phase, whose tables hold every call that a
+// buffer layout admits.
 static bool fused_fits(const DgmMoeArgs* A) {
-  const bool big = A->act_format != DGM_ACT_QOQ && A->act_format != DGM_ACT_NVFP4 && !A->fe_in_mega;
-  return A->num_tokens * A->topk <= (big ? FUSED_BIG_ROUTES : FUSED_MAX_ROUTES) && A->num_local_experts <= FUSED_MAX_LOCAL &&
-         A->num_tokens <= (big ? FUSED_BIG_ROUTES : FUSED_MAX_TOKENS) && A->hidden / 64 <= FUSED_MAX_NB64;
+  return A->num_tokens * A->topk <= FUSED_MAX_ROUTES && A->num_local_experts <= FUSED_MAX_LOCAL &&
+         A->num_tokens <= FUSED_MAX_TOKENS && A->hidden / 64 <= FUSED_MAX_NB64;
 }
-
 // One launch of the persistent kernel running `phases` (FusedParams::phases) of the layer, with
 // the buffer's own workspace views.
 static int fused_launch_phases(const DgmMoeArgs* A, int phases, hipStream_t stream) {
@@ -975,7 +576,8 @@ int dgm_fused_launch_ws(const DgmMoeArgs* A, int phases, const DgmWorkspace& w, 
   uint8_t* buf = (uint8_t*)A->buffer;
   {
     const int fast = (A->fe_flags & DGM_FE_FORCE_BALANCED) ? SELECT_IN_MEGA_FAST_BALANCED : SELECT_IN_MEGA_FAST_TOKENS;
-    const bool sel = (A->fe_in_mega || (A->select_in_mega && A->num_tokens <= fast)) && (phases & 1);
+    // (the large-batch form reads the top-k)
+    const bool sel = (A->fe_in_mega || (A->select_in_mega && A->num_tokens <= fast)) && (phases & 1) && fused_fits(A);
     if (A->select_in_mega && !sel && (phases & 1)) {
       int st = materialize_topk(A, buf, L, stream);
       if (st) return st;
@@ -1060,39 +662,14 @@ int dgm_megamoe_split_launch(const DgmMoeArgs* A, hipStream_t stream) {
   }
   const DgmBufferLayout* L = A->layout;
   DGM_CHECK_ARG(A->num_tokens >= 0 && (int64_t)A->num_tokens * A->topk <= L->max_routes, "num_tokens exceeds the buffer");
+  DGM_CHECK_ARG(A->num_local_experts > 0 && A->num_local_experts <= FUSED_BIG_LOCAL, "num_local_experts");
   if (A->num_tokens == 0) return 0;
-  uint8_t* buf = (uint8_t*)A->buffer;
-  const int routes_n = A->num_tokens * A->topk;
-  if (A->select_in_mega) {
-    int st0 = materialize_topk(A, buf, L, stream);
-    if (st0) return st0;
-  }
-  hipLaunchKernelGGL(k_dispatch, dim3(1), dim3(DISPATCH_THREADS), 0, stream,
-                     (const int64_t*)(buf + L->topk_idx), routes_n, A->expert_begin, A->num_local_experts,
-                     buf + L->pool, A->recv_stats);
-  int st = dgm_last_launch_status();
-  if (st) return st;
-  const int KT1 = A->hidden / 128, KT2 = A->intermediate / 128;
-#define DGM_SPLIT(K1, K2)                                                                       \
-  (A->act_format == DGM_ACT_MXFP4   ? launch_experts<K1, K2, DGM_ACT_MXFP4>(A, buf, L, stream)   \
-   : A->act_format == DGM_ACT_MXFP8 ? launch_experts<K1, K2, DGM_ACT_MXFP8>(A, buf, L, stream)   \
-                                    : launch_experts<K1, K2, DGM_ACT_FP8F128>(A, buf, L, stream))
-  if (KT1 == 24 && KT2 == 10) {
-    st = DGM_SPLIT(24, 10);
-  } else if (KT1 == 4 && KT2 == 2) {
-    st = DGM_SPLIT(4, 2);
-  } else if (KT1 == 8 && KT2 == 4) {
-    st = DGM_SPLIT(8, 4);
-  } else {
-    DGM_CHECK_ARG(false, "supported (hidden, intermediate): (3072, 1280), (512, 256), (1024, 512)");
-  }
-#undef DGM_SPLIT
-  if (st) return st;
-  dim3 cg((A->hidden / 4 + 255) / 256, A->num_tokens);
-  hipLaunchKernelGGL(k_combine, cg, dim3(256), 0, stream, (const uint16_t*)(buf + L->partials), L->max_tokens,
-                     (const int64_t*)(buf + L->topk_idx), A->num_tokens, A->hidden, A->topk, A->expert_begin,
-                     A->num_local_experts, (uint16_t*)A->y);
-  return dgm_last_launch_status();
+  // the persistent kernel twice (dispatch + L1, then L2), then the combine: no launch has a wait
+  // on another workgroup, so none needs its grid resident at once (E384, 257 tokens, FP8F128:
+  // 389 us; with the launches this replaced, see FORM_BIG, 989 us)
+  int st = fused_launch_phases(A, 1, stream);
+  if (!st) st = fused_launch_phases(A, 2 | 4, stream);
+  return st ? st : launch_combine(A, (uint8_t*)A->buffer, L, stream);
 }
 
 }  // extern "C"

@@ -1,5 +1,5 @@
-"""The persistent kernel's large-batch form (more than 1024 routes or 256 tokens; MXFP4, MXFP8 and
-FP8F128 activations) against the plain form: a token's output does not depend on the tokens beside
+"""The persistent kernel's large-batch form (more than 1024 routes, 256 tokens or 512 local experts;
+MXFP4, MXFP8 and FP8F128 activations) against the plain form: a token's output does not depend on the tokens beside
 it, so y of one large call equals, bit for bit, y of the same tokens in calls small enough for the
 plain form. Its dispatch table against the oracle's, and the recv stats against the counts."""
 import os
@@ -101,3 +101,55 @@ def test_large_batch_equals_small_calls(case, fmt):
         ys, _, bs = _call(dgm, x[t:t + n], idx[t:t + n], w[t:t + n], l1, l2, fmt, n, E, topk, H, I, ep, rank)
         assert dgm.mega.fused_last_form(bs) == 0
         assert torch.equal(ys.view(torch.int16), y[t:t + n].view(torch.int16)), t
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", ["mxfp4", "mxfp8"])
+@pytest.mark.parametrize("split", [False, True])
+def test_many_local_experts_equal_the_routed_ones(fmt, split):
+    """1000 local experts (few tokens, top-k left to the layer call): the same y as a layer that
+    holds only the routed experts, renumbered."""
+    need_gpu()
+    import hopper_megamoe_basedondeepgemm_amd as dgm
+    M, topk, E, H, I = 7, 8, 1000, 512, 256
+    print(f"1000 local experts {fmt} split={split}", flush=True)
+    l1, l2 = _weights(dgm, E, H, I, 5)
+    g = torch.Generator(device="cuda").manual_seed(6)
+    x = torch.randn((M, H), generator=g, device="cuda").bfloat16()
+    rw = (torch.randn((E, H), generator=g, device="cuda") / 20).bfloat16()
+    buf = dgm.get_fused_symm_buffer_for_mega_moe(None, E, M, topk, H, I, act_format=fmt)
+    dgm.fable_router_quant_topk_frontend(x, rw, buf, select_in_mega=True)
+    y = torch.full((M, H), 7.0, dtype=torch.bfloat16, device="cuda")
+    stats = torch.zeros(E, dtype=torch.int32, device="cuda")
+    dgm.mega._fused(y, l1, l2, buf, stats, 10.0, split=split)
+    torch.cuda.synchronize()
+    assert buf.kernel_error() == 0 and dgm.mega.fused_last_form(buf) == 4
+    idx = buf.topk_idx[:M].cpu().numpy()
+    counts, active, offs, routes = moe.dispatch(idx, 0, E)
+    for got, want in zip(buf.pool_table(), (counts, active, offs, routes)):
+        np.testing.assert_array_equal(got.numpy(), want)
+    np.testing.assert_array_equal(stats.cpu().numpy(), counts)
+    act = torch.from_numpy(active).cuda()
+    sub = [tuple(t[act].contiguous() if t is not None else None for t in l) for l in (l1, l2)]
+    ys, _, bs = _call(dgm, x, np.searchsorted(active, idx), buf.topk_weights[:M].cpu().numpy(), sub[0], sub[1], fmt, M,
+                      len(active), topk, H, I, 1, 0)
+    assert dgm.mega.fused_last_form(bs) == 0
+    assert torch.equal(ys.view(torch.int16), y.view(torch.int16))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", ["mxfp4", "mxfp8", "fp8f128"])
+def test_split_launches_equal_one_launch(fmt):
+    """The plain form as L1, L2 and combine launches: y of the one launch bit for bit, with a token
+    of one local route (written by L2 itself in the one launch), unrouted tokens and ragged slabs."""
+    need_gpu()
+    import hopper_megamoe_basedondeepgemm_amd as dgm
+    M, topk, E, ep, H, I = 90, 4, 16, 2, 1024, 512
+    print(f"split launches {fmt}", flush=True)
+    rng = np.random.default_rng(9)
+    l1, l2 = _weights(dgm, E // ep, H, I, 8)
+    x = torch.randn((M, H), generator=torch.Generator(device="cuda").manual_seed(9), device="cuda").bfloat16()
+    idx, w = _routing("uneven", rng, M, E, topk)
+    outs = [_call(dgm, x, idx, w, l1, l2, fmt, M, E, topk, H, I, ep, 0, split=sp)[:2] for sp in (False, True)]
+    assert torch.equal(outs[0][0].view(torch.int16), outs[1][0].view(torch.int16))
+    assert torch.equal(outs[0][1], outs[1][1])
