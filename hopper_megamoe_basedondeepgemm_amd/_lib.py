@@ -30,6 +30,7 @@ EXPORTS = [
     "dgm_reorder_fp4_nibbles", "dgm_untransform_fp4_weights", "dgm_untransform_nvfp4_weights",
     "dgm_router_logits_topk_launch", "dgm_router_topk_launch_stamped", "dgm_frontend_workgroups",
     "dgm_quantize_mxfp4_typed", "dgm_quantize_nvfp4_typed", "dgm_quantize_qoq_typed", "dgm_quantize_qoq_int4_typed",
+    "dgm_transform_qoq_weights_checked", "dgm_transform_qoq_int4_weights_checked",
 ]
 # source element types of the weight packers (DGM_SRC_*)
 SRC_DTYPES = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
@@ -103,6 +104,8 @@ def load():
         "dgm_quantize_qoq": ([vp, i64, i64, vp, vp, vp, vp, vp], i32),
         "dgm_quantize_qoq_int4": ([vp, i64, i64, vp, vp, vp], i32),
         "dgm_transform_qoq_int4_weights": ([vp, vp, i32, i32, i32, i32, vp, vp, vp, vp], i32),
+        "dgm_transform_qoq_weights_checked": ([vp, vp, vp, vp, i32, i32, i32, i32, vp, vp, vp, vp, vp], i32),
+        "dgm_transform_qoq_int4_weights_checked": ([vp, vp, i32, i32, i32, i32, vp, vp, vp, vp, vp], i32),
         "dgm_cast_int8_rows": ([vp, i64, i64, vp, vp, vp], i32),
         "dgm_transform_fp4_weights": ([vp, vp, i32, i32, i32, i32, i32, vp, vp, vp], i32),
         "dgm_fused_buffer_layout": ([i32, i32, i32, i32, i32, i32, i32, ctypes.POINTER(BufferLayout)], i32),

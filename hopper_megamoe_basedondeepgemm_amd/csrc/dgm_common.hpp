@@ -80,7 +80,22 @@ DGM_DEV float e8m0_inv(uint32_t code) {
 }
 // ceil(fp32(log2(x))) with log2 evaluated in double and rounded once to fp32: the
 // behaviour of the log2-based scale rules near powers of two.
-DGM_DEV float ceil_log2_f32(float x) { return ceilf((float)log2((double)x)); }
+// For a normal x = 2^k (1 + f 2^-23) that is k at f = 0 and k + 1 at f >= 64 (log2 is then at least
+// 1.1e-5 above k, and fp32 values up to 128 are at most 7.7e-6 apart); only the mantissas between,
+// where the rounding to fp32 may fall back to k, take the double logarithm.
+DGM_DEV float ceil_log2_f32(float x) {
+  const uint32_t u = __float_as_uint(x), f = u & 0x7fffffu;
+  if (u - 0x00800000u < 0x7f000000u && (f == 0u || f >= 64u)) return (float)((int)(u >> 23) - (f == 0u ? 127 : 126));
+  return ceilf((float)log2((double)x));
+}
+// floor(fp32(log2(x))), likewise: for x = 2^k (1 + f 2^-23) with |k| <= 15 the rounding reaches k + 1
+// only from f > 2^23 - 64 on.
+DGM_DEV float floor_log2_f32(float x) {
+  const uint32_t u = __float_as_uint(x), f = u & 0x7fffffu;
+  const int k = (int)(u >> 23) - 127;
+  if (k >= -15 && k <= 15 && f <= 0x7fffffu - 64u) return (float)k;
+  return floorf((float)log2((double)x));
+}
 
 // ---------------------------------------------------------------- E4M3 (OCP fn)
 // fp32 -> e4m3fn byte, round to nearest even; anything rounding above 448 -> 0x7F (NaN).
@@ -128,6 +143,20 @@ DGM_DEV float key_value(uint32_t key) {
   uint32_t o = key >> 16;
   uint32_t b = (o & 0x8000u) ? (o & 0x7fffu) : (~o & 0xffffu);
   return bf16_to_f32((uint16_t)b);
+}
+
+// Maximum (or minimum) over aligned groups of 2, 4 or 16 lanes, in every lane of the group (fmaxf /
+// fminf: a NaN is passed over). Lanes of a group must all be active.
+template <int CTRL>
+DGM_DEV float dpp_f32(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, false));
+}
+DGM_DEV float max_lanes2(float v) { return fmaxf(v, dpp_f32<0xB1>(v)); }                          // quad_perm [1,0,3,2]
+DGM_DEV float max_lanes4(float v) { v = max_lanes2(v); return fmaxf(v, dpp_f32<0x4E>(v)); }       // quad_perm [2,3,0,1]
+DGM_DEV float max_lanes16(float v) {
+  v = max_lanes4(v);
+  v = fmaxf(v, dpp_f32<0x141>(v));            // row_half_mirror
+  return fmaxf(v, dpp_f32<0x140>(v));         // row_mirror
 }
 
 // Wave-wide max, uniform result: DPP within rows of 16 lanes (quad xor 1, quad xor 2, half

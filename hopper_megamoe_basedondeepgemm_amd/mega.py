@@ -181,7 +181,7 @@ def transform_mxfp4_weights_for_mega_moe_fused(l1, l2, src_order="marlin"):
     return _transform_one(l1[0], l1[1], True, so), _transform_one(l2[0], l2[1], False, so)
 
 
-def _transform_qoq_one(q, l1_interleave):
+def _transform_qoq_one(q, l1_interleave, bad):
     packed, s2, z, s1 = q
     _lib.require_gpu(packed, s2, z, s1)
     assert packed.dtype == torch.uint8 and s2.dtype == torch.uint8 and z.dtype == torch.uint8
@@ -190,17 +190,16 @@ def _transform_qoq_one(q, l1_interleave):
     K = Kh * 2
     assert s2.shape == (E, N, K // 128) and z.shape == (E, N, K // 128) and s1.shape == (E, N)
     assert N % 16 == 0 and K % 128 == 0, (N, K)
-    # the fused layout keeps z and s2 as one nibble each (quantize_to_qoq: z 0..15, s2 1..15)
-    if int(torch.maximum(s2.max(), z.max()).item()) > 15:
-        raise ValueError("QoQ meta out of range: z and s2 must be < 16")
     KT, NB = K // 128, N // 16
     vals = torch.empty((E, NB, KT, 64, 16), dtype=torch.uint8, device=packed.device)
     meta = torch.empty((E, NB, KT, 16), dtype=torch.uint8, device=packed.device)
     rs = torch.empty((E, N), dtype=torch.float32, device=packed.device)
-    _lib.check(_lib.load().dgm_transform_qoq_weights(
+    # the fused layout keeps z and s2 as one nibble each (quantize_to_qoq: z 0..15, s2 1..15): the
+    # transform flags any that do not fit in ``bad``
+    _lib.check(_lib.load().dgm_transform_qoq_weights_checked(
         _lib.ptr(packed.contiguous()), _lib.ptr(s2.contiguous()), _lib.ptr(z.contiguous()),
         _lib.ptr(s1.contiguous()), E, N, K, int(l1_interleave), _lib.ptr(vals), _lib.ptr(meta), _lib.ptr(rs),
-        _lib.stream()))
+        _lib.ptr(bad), _lib.stream()))
     return vals, meta, rs
 
 
@@ -210,7 +209,11 @@ def transform_qoq_weights_for_mega_moe_fused(l1, l2):
     Returns ``((w1_values, w1_meta, w1_s1), (w2_values, w2_meta, w2_s1))``: 4-bit codes in
     int8 matrix-core fragment order, per (row, K128) zero points and group scales, per-row
     scales. Invariant: dequant(transform(q)) == interleave(dequant(q))."""
-    return _transform_qoq_one(l1, True), _transform_qoq_one(l2, False)
+    bad = torch.zeros(1, dtype=torch.int32, device=l1[0].device)
+    out = _transform_qoq_one(l1, True, bad), _transform_qoq_one(l2, False, bad)
+    if bad.item():        # (one wait for both matrices)
+        raise ValueError("QoQ meta out of range: z and s2 must be < 16")
+    return out
 
 
 def _transform_nvfp4_one(packed, scale, l1_interleave, src_order):
@@ -239,23 +242,20 @@ def transform_nvfp4_weights_for_mega_moe_fused(l1, l2, src_order="marlin"):
     return _transform_nvfp4_one(*l1, True, src_order), _transform_nvfp4_one(*l2, False, src_order)
 
 
-def _transform_qoq_int4_one(q, l1_interleave):
+def _transform_qoq_int4_one(q, l1_interleave, bad):
     packed, plane = q
     _lib.require_gpu(packed, plane)
     assert packed.dtype == torch.uint8 and plane.dtype == torch.int32 and packed.dim() == 3
     E, N, Kh = packed.shape
     K = Kh * 2
     assert tuple(plane.shape) == (E, N, K // 128) and N % 16 == 0 and K % 128 == 0, (plane.shape, packed.shape)
-    # the fused layout keeps z and s2 as one nibble each (quantize_to_qoq_int4: z <= 15, s2 <= 15)
-    pl = plane.contiguous()
-    if int(torch.maximum(pl & 0xFF, (pl >> 8) & 0xFF).max().item()) > 15:
-        raise ValueError("QoQ plane out of range: z and s2 must be < 16")
     vals = torch.empty((E, N // 16, K // 128, 64, 16), dtype=torch.uint8, device=packed.device)
     meta = torch.empty((E, N // 16, K // 128, 16), dtype=torch.uint8, device=packed.device)
     rs = torch.empty((E, N), dtype=torch.float32, device=packed.device)
-    _lib.check(_lib.load().dgm_transform_qoq_int4_weights(
-        _lib.ptr(packed.contiguous()), _lib.ptr(pl), E, N, K, int(l1_interleave), _lib.ptr(vals), _lib.ptr(meta),
-        _lib.ptr(rs), _lib.stream()))
+    # (z <= 15 and s2 <= 15 from quantize_to_qoq_int4, flagged as above)
+    _lib.check(_lib.load().dgm_transform_qoq_int4_weights_checked(
+        _lib.ptr(packed.contiguous()), _lib.ptr(plane.contiguous()), E, N, K, int(l1_interleave), _lib.ptr(vals),
+        _lib.ptr(meta), _lib.ptr(rs), _lib.ptr(bad), _lib.stream()))
     return vals, meta, rs
 
 
@@ -264,7 +264,11 @@ def transform_qoq_int4_weights_for_mega_moe_sm90(l1_weights, l2_weights, block_n
     plane int32 [E, N, K/128])`` -> the same layout as ``transform_qoq_weights_for_mega_moe_fused``
     (values, meta, s1) per matrix. ``block_n`` picks an SM90 tile there and has no effect here."""
     assert block_n in (128, 256)
-    return _transform_qoq_int4_one(l1_weights, True), _transform_qoq_int4_one(l2_weights, False)
+    bad = torch.zeros(1, dtype=torch.int32, device=l1_weights[0].device)
+    out = _transform_qoq_int4_one(l1_weights, True, bad), _transform_qoq_int4_one(l2_weights, False, bad)
+    if bad.item():
+        raise ValueError("QoQ plane out of range: z and s2 must be < 16")
+    return out
 
 
 def transform_weights_for_mega_moe(l1, l2):

@@ -168,6 +168,15 @@ int dgm_quantize_qoq_int4(const void* w_bf16, int64_t rows, int64_t K, void* pac
 int dgm_transform_qoq_int4_weights(const void* packed, const void* plane_i32, int E, int N, int K, int l1_interleave,
                                    void* dst_values, void* dst_meta, void* dst_s1, hipStream_t stream);
 
+/* The two transforms above with the range check of the values they narrow: *out_of_range (a device
+ * word the caller has cleared; NULL: unchecked) is set to 1 when a z or s2 exceeds 15. */
+int dgm_transform_qoq_weights_checked(const void* packed, const void* s2, const void* z, const void* s1, int E, int N,
+                                      int K, int l1_interleave, void* dst_values, void* dst_meta, void* dst_s1,
+                                      int* out_of_range, hipStream_t stream);
+int dgm_transform_qoq_int4_weights_checked(const void* packed, const void* plane_i32, int E, int N, int K,
+                                           int l1_interleave, void* dst_values, void* dst_meta, void* dst_s1,
+                                           int* out_of_range, hipStream_t stream);
+
 /* ------------------------------------------------------------------ fused buffer
  * Replaces csrc/apis/mega_fused.hpp:31-76 get_symm_buffer_size_for_fused_mega_moe:
  * byte offsets of every view inside one device buffer (single GPU, no symmetric memory). */
