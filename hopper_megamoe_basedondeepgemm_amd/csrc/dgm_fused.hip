@@ -526,171 +526,119 @@ DGM_DEV bool spin_until2(const int* p, int target, int limit, int* err, int* her
   }
 }
 
-// Stage the B slab (16 columns = rows row_of(c) of a [rows, KT*128] activation matrix with
-// row_bytes and per-32 E8M0 scales) into LDS in fragment order. Column c >= n is zero.
-// COHERENT: the rows were written by other workgroups of this launch (agent-scope loads).
-template <int KT, int ACT, bool COHERENT, class S, class RowOf>
-DGM_DEV void stage_slab(S& s, const uint8_t* __restrict__ src, const uint8_t* __restrict__ ssrc,
-                        int row_bytes, int n, RowOf row_of) {
-  // (the thread index made opaque: the addresses below are computed here, not hoisted out of
-  // the item loop and kept live, or spilled, across it)
-  int tid = threadIdx.x;
-  asm volatile("" : "+v"(tid));
-  for (int f = tid; f < KT * 64; f += FT) {
-    const int kt = f >> 6, l = f & 63, c = l & 15;
-    uint4 v0 = make_uint4(0, 0, 0, 0), v1 = make_uint4(0, 0, 0, 0);
-    if (c < n) {
-      const size_t r = (size_t)row_of(c);
-      // E2M1: 16 bytes at K = 32 g; E4M3: K = 16 g .. +16 and K = 64 + 16 g .. +16 (g = l / 16)
-      const uint8_t* q = ACT == DGM_ACT_MXFP4 ? src + r * row_bytes + kt * 64 + (l >> 4) * 16
-                                              : src + r * row_bytes + kt * 128 + (l >> 4) * 16;
-      if (COHERENT) {
-        uint64_t a0 = ld_agent64(q), a1 = ld_agent64(q + 8);
-        v0 = make_uint4((uint32_t)a0, (uint32_t)(a0 >> 32), (uint32_t)a1, (uint32_t)(a1 >> 32));
-        if (ACT != DGM_ACT_MXFP4) {
-          uint64_t b0 = ld_agent64(q + 64), b1 = ld_agent64(q + 72);
-          v1 = make_uint4((uint32_t)b0, (uint32_t)(b0 >> 32), (uint32_t)b1, (uint32_t)(b1 >> 32));
-        }
-      } else {
-        v0 = *reinterpret_cast<const uint4*>(q);
-        if (ACT != DGM_ACT_MXFP4) v1 = *reinterpret_cast<const uint4*>(q + 64);
-      }
-    }
-    uint4* dst = reinterpret_cast<uint4*>(&s.bst[kt][l][0]);
-    dst[0] = v0;
-    if (ACT != DGM_ACT_MXFP4) dst[S::BV - 1] = v1;
-  }
-  for (int f = tid; f < ((KT + 3) / 4) * 64; f += FT) {
-    const int g = f >> 6, l = f & 63, c = l & 15;
-    uint32_t w = 0x7f7f7f7fu;
-    if (c < n) {
-      const size_t r = (size_t)row_of(c);
-      w = 0;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int kt = 4 * g + j;
-        uint32_t b = 127u;
-        if (kt < KT) {
-          const uint8_t* q = ssrc + r * (KT * 4) + kt * 4 + (l >> 4);
-          b = COHERENT ? ld_agent8(q) : (uint32_t)*q;
-        }
-        w |= b << (8 * j);
-      }
-    }
-    s.bsc[g][l] = w;
-  }
-}
-
-// A B slab held in registers between its loads and its LDS stores (the loads are issued
-// early, ahead of the weight tiles they must not queue behind). Same fragments as stage_slab.
-// Values are kept exactly as loaded (vectors, or the 64-bit halves of agent-scope loads) and
-// only combined or masked at the store: doing either earlier would wait for every older load.
-// Every lane loads (from row 0 when it has no row), so no loaded value crosses a divergent
-// branch.
+// A B slab (16 columns = rows row_of(c) of an activation matrix, in matrix-core fragment order) on
+// its way to LDS: held in registers between its loads and its LDS stores (the loads are issued
+// early, ahead of the weight tiles they must not queue behind). Values are kept exactly as loaded
+// (vectors, or the 64-bit halves of agent-scope loads) and only combined at the store: doing it
+// earlier would wait for every older load.
+// Only the n columns with a row are loaded and stored: a matrix-core column depends on its own B
+// column alone, so what the others hold (an earlier slab, or nothing) reaches no result. The
+// fragments (K-tile kt, column c, lane group g) are dealt out as f = (kt n + c) 4 + g to thread
+// f % 512: with one or two routes per expert, one or two waves load and store a slab and the rest
+// skip it. (Against fixed columns per lane, the empty ones stored as zeros by every wave: QoQ at 16
+// tokens 126.1 -> 122.1 us, A-MXFP8 at 8 tokens 75.3 -> 74.7, A-MXFP8 at 512 448 -> 446; NVFP4 at 64
+// tokens 345.0 -> 343.9; 2 to 13 VGPRs fewer.)
 template <int KT, int ACT, bool COHERENT, bool MIDL = COHERENT>
 struct SlabRegs {
   static constexpr int FR = (KT * 64 + FT - 1) / FT;
   v4u v0[FR], v1[FR];            // non-coherent fragments
   uint64_t h[FR][4];             // coherent fragments: 64-bit halves (K bytes 0-15, 64-79)
-  uint32_t sb[4];                // scale dwords of K-tiles 4g .. 4g+3 (byte l/16 is this lane's)
-  uint32_t ok;                   // bit j: fragment j holds a real row; bit 8 + j: scale byte j
+  uint32_t sb[4];                // MXFP, FP8F128: the four dwords of scale unit (c, gs): K-tiles 4 gs .. +3
   float fsc;                     // QoQ input rows: the token's scale (threads 0-15)
-  uint64_t sc2[FR];              // QoQ intermediate rows: fragment j's two chunk scales (lanes 0-15)
+  uint64_t sc2[FR];              // QoQ intermediate rows: fragment j's two chunk scales (lane group 0)
   uint32_t s16[FR];              // NVFP4: the dword holding fragment j's two 16-block scales
   float w;
+  int n;                         // columns with a row
+  uint32_t nm;                   // slab_magic(n)
 };
+// Fragment f of an n-column slab: its K-tile, column and lane group (f < 64 KT <= 1536, n <= 16: the
+// quotient by n as a product with ceil(2^16 / n), exact since f / 4 * n < 2^16).
+struct SlabFrag { int kt, c, g; };
+DGM_DEV SlabFrag slab_frag(int f, int n, uint32_t nm) {
+  const int m = f >> 2, kt = (int)(((uint32_t)m * nm) >> 16);
+  return SlabFrag{kt, m - kt * n, f & 3};
+}
+DGM_DEV uint32_t slab_magic(int n) { return (0x10000u + (uint32_t)n - 1u) / (uint32_t)n; }
 
 // COHERENT: agent-scope loads (rows written by other workgroups of this launch); MIDL: the
-// intermediate rows' layout (QoQ: per-chunk scales) rather than the input activations'.
+// intermediate rows' layout (QoQ: per-chunk scales) rather than the input activations'. n_ >= 1.
 template <int KT, int ACT, bool COHERENT, bool MIDL, class RowOf, class WeightOf>
 DGM_DEV void slab_load(SlabRegs<KT, ACT, COHERENT, MIDL>& r, const uint8_t* __restrict__ src, const uint8_t* __restrict__ ssrc,
-                       int row_bytes, int n, RowOf row_of, WeightOf weight_of) {
+                       int row_bytes, int n_, RowOf row_of, WeightOf weight_of) {
   const int tid = threadIdx.x;
-  uint32_t ok = 0;
-  // MASK: only the lanes whose column holds a real row load (the slab store zeroes the others):
-  // with one route per expert, 15 of 16 columns are empty, and their loads (of row 0) kept the
-  // memory pipeline busy for ~0.7 us at each workgroup's first slab (A-MXFP, FP8F128: 0.4-1.7
-  // us per layer call). QoQ and NVFP4 keep the unconditional loads: with the branches their
-  // kernels spill more registers (5 and 9 values) and measured slower.
-  constexpr bool MASK = ACT == DGM_ACT_MXFP4 || ACT == DGM_ACT_MXFP8 || ACT == DGM_ACT_FP8F128;
+  const int n = __builtin_amdgcn_readfirstlane(n_ < 16 ? n_ : 16);
+  const uint32_t nm = slab_magic(n);
+  r.n = n;
+  r.nm = nm;
 #pragma unroll
   for (int j = 0; j < SlabRegs<KT, ACT, COHERENT, MIDL>::FR; ++j) {
     const int f = tid + j * FT;
-    const int l = f & 63, c = l & 15;
-    const bool have = f < KT * 64 && c < n;
-    ok |= have ? 1u << j : 0u;
-    const int kt = have ? f >> 6 : 0;
-    const size_t rr = have ? (size_t)row_of(c) : 0;
-    // E2M1 (MXFP4, NVFP4): 16 bytes at K = 32 g; E4M3 / int8: K = 16 g .. +16 and
-    // K = 64 + 16 g .. +16 (g = l / 16)
-    constexpr bool FP4 = ACT == DGM_ACT_MXFP4 || ACT == DGM_ACT_NVFP4;
-    const uint8_t* q = FP4 ? src + rr * row_bytes + kt * 64 + (l >> 4) * 16
-                           : src + rr * row_bytes + kt * 128 + (l >> 4) * 16;
-    if (COHERENT) {
+    if constexpr (COHERENT) {
       r.h[j][0] = r.h[j][1] = r.h[j][2] = r.h[j][3] = 0;
-      if (!MASK || have) {
+    } else {
+      r.v0[j] = r.v1[j] = v4u{0u, 0u, 0u, 0u};
+    }
+    r.s16[j] = 0u;
+    r.sc2[j] = 0;
+    if (f < n * KT * 4) {
+      const SlabFrag F = slab_frag(f, n, nm);
+      const size_t rr = (size_t)row_of(F.c);
+      // E2M1 (MXFP4, NVFP4): 16 bytes at K = 32 g; E4M3 / int8: K = 16 g .. +16 and
+      // K = 64 + 16 g .. +16
+      constexpr bool FP4 = ACT == DGM_ACT_MXFP4 || ACT == DGM_ACT_NVFP4;
+      const uint8_t* q = src + rr * row_bytes + F.kt * (FP4 ? 64 : 128) + F.g * 16;
+      if constexpr (COHERENT) {
         r.h[j][0] = ld_agent64(q);
         r.h[j][1] = ld_agent64(q + 8);
-        if (!FP4) {
+        if constexpr (!FP4) {
           r.h[j][2] = ld_agent64(q + 64);
           r.h[j][3] = ld_agent64(q + 72);
         }
-      }
-    } else {
-      r.v0[j] = r.v1[j] = v4u{0u, 0u, 0u, 0u};
-      if (!MASK || have) {
+      } else {
         r.v0[j] = *reinterpret_cast<const v4u*>(q);
-        if (!FP4) r.v1[j] = *reinterpret_cast<const v4u*>(q + 64);
+        if constexpr (!FP4) r.v1[j] = *reinterpret_cast<const v4u*>(q + 64);
       }
-    }
-    if constexpr (ACT == DGM_ACT_NVFP4) {
-      // the two E4M3 scales of the fragment (16-blocks 8 kt + 2 g, +1; row pitch KT * 8 bytes),
-      // as the aligned dword holding them
-      const uint32_t* sq = reinterpret_cast<const uint32_t*>(ssrc + rr * (KT * 8) + ((8 * kt + 2 * (l >> 4)) & ~3));
-      r.s16[j] = COHERENT ? __hip_atomic_load(sq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *sq;
+      if constexpr (ACT == DGM_ACT_NVFP4) {
+        // the two E4M3 scales of the fragment (16-blocks 8 kt + 2 g, +1; row pitch KT * 8 bytes),
+        // as the aligned dword holding them
+        const uint32_t* sq = reinterpret_cast<const uint32_t*>(ssrc + rr * (KT * 8) + ((8 * F.kt + 2 * F.g) & ~3));
+        r.s16[j] = COHERENT ? __hip_atomic_load(sq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *sq;
+      }
+      if constexpr (ACT == DGM_ACT_QOQ && MIDL) {
+        // intermediate rows: fp32 scale per 64-K chunk (row pitch KT * 8 bytes)
+        if (F.g == 0) r.sc2[j] = ld_agent64(ssrc + rr * (KT * 8) + F.kt * 8);
+      }
     }
   }
   constexpr int KG = (KT + 3) / 4;
-  static_assert(KG * 64 <= FT, "one scale word per thread");
-  if constexpr (ACT == DGM_ACT_NVFP4) {
-    // (scales loaded with the fragments)
-  } else if constexpr (ACT == DGM_ACT_QOQ) {
-    if (MIDL) {
-      // intermediate rows: fp32 scale per 64-K chunk (row pitch KT * 8 bytes); lane l < 16 of
-      // fragment j (K-tile kt, column l) loads the two chunk scales of its tile
-#pragma unroll
-      for (int j = 0; j < SlabRegs<KT, ACT, COHERENT, MIDL>::FR; ++j) {
-        const int f = tid + j * FT;
-        const bool have = (ok >> j) & 1u && (f & 63) < 16;
-        const size_t rr = have ? (size_t)row_of(f & 15) : 0;
-        r.sc2[j] = ld_agent64(ssrc + rr * (KT * 8) + (have ? (f >> 6) * 8 : 0));
+  static_assert(16 * KG <= FT, "one scale unit per thread");
+  if constexpr (ACT == DGM_ACT_QOQ) {
+    // input rows: one fp32 scale per token (row pitch KT * 4 bytes: the reference's [M, K/128]
+    // copies), thread c < 16
+    if constexpr (!MIDL) {
+      r.fsc = 0.f;
+      if (tid < n) {
+        const float* fq = reinterpret_cast<const float*>(ssrc + (size_t)row_of(tid) * (KT * 4));
+        r.fsc = COHERENT ? __hip_atomic_load(fq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *fq;
       }
-    } else {
-      // input rows: one fp32 scale per token (row pitch KT * 4 bytes: the reference's
-      // [M, K/128] copies), thread c < 16
-      const int c = tid & 15;
-      const bool have = tid < 16 && c < n;
-      const size_t rr = have ? (size_t)row_of(c) : 0;
-      const float* fq = reinterpret_cast<const float*>(ssrc + rr * (KT * 4));
-      r.fsc = COHERENT ? __hip_atomic_load(fq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *fq;
-      ok |= have ? 1u << 8 : 0u;
     }
-  } else {
-    const int g = tid >> 6, l = tid & 63, c = l & 15;
-    const bool have = tid < KG * 64 && c < n;
-    const size_t rr = have ? (size_t)row_of(c) : 0;
+  } else if constexpr (ACT != DGM_ACT_NVFP4) {
+    // scale unit (column c, scale dword gs), from the last thread down: beside the fragments
+    const int u = FT - 1 - tid, c = u / KG, gs = u % KG;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int kt = 4 * g + j;
-      const bool hb = have && kt < KT;
-      ok |= hb ? 1u << (8 + j) : 0u;
-      const uint32_t* q = reinterpret_cast<const uint32_t*>(ssrc + (hb ? rr * (KT * 4) + kt * 4 : 0));
-      r.sb[j] = 0u;
-      if (!MASK || hb) r.sb[j] = COHERENT ? __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *q;
+    for (int j = 0; j < 4; ++j) r.sb[j] = 0x7f7f7f7fu;
+    if (c < n) {
+      const uint8_t* q = ssrc + (size_t)row_of(c) * (KT * 4) + gs * 16;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (4 * gs + j < KT) {
+          const uint32_t* d = reinterpret_cast<const uint32_t*>(q + 4 * j);
+          r.sb[j] = COHERENT ? __hip_atomic_load(d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *d;
+        }
     }
   }
-  r.ok = ok;
-  r.w = tid < n && tid < 16 ? weight_of(tid) : 0.f;
+  r.w = 0.f;
+  if (tid < n) r.w = weight_of(tid);
 }
 
 template <int KT, int ACT, bool COHERENT, bool MIDL, class S>
@@ -699,31 +647,28 @@ DGM_DEV void slab_store(S& s, const SlabRegs<KT, ACT, COHERENT, MIDL>& r) {
   // rather than hoisted out of the work loop and kept live, or spilled, across it)
   int tid = threadIdx.x;
   asm volatile("" : "+v"(tid));
-  const v4u z = {0u, 0u, 0u, 0u};
-  if constexpr (ACT == DGM_ACT_NVFP4) {
-    // fragment (K-tile kt, column c, 32-K chunk g') -> f16 operand of op g' for the four lane
-    // groups q (K = 32 g' + 8 q .. +8): E2M1 -> f16 exactly, times the E4M3 block scale (the
-    // products are exact in f16)
+  const int n = r.n;
+  const uint32_t nm = r.nm;
 #pragma unroll
-    for (int j = 0; j < SlabRegs<KT, ACT, COHERENT, MIDL>::FR; ++j) {
-      const int f = tid + j * FT;
-      if (f < KT * 64) {
-        const bool have = (r.ok >> j) & 1u;
-        const int kt = f >> 6, l = f & 63, c = l & 15, gq = l >> 4;
-        uint32_t w[4];
-        if (COHERENT) {
-          w[0] = (uint32_t)r.h[j][0];
-          w[1] = (uint32_t)(r.h[j][0] >> 32);
-          w[2] = (uint32_t)r.h[j][1];
-          w[3] = (uint32_t)(r.h[j][1] >> 32);
-        } else {
-          w[0] = r.v0[j].x;
-          w[1] = r.v0[j].y;
-          w[2] = r.v0[j].z;
-          w[3] = r.v0[j].w;
-        }
-        const uint32_t sc2 = r.s16[j] >> ((gq & 1) * 16);      // byte 0: block 2 g', byte 1: 2 g' + 1
+  for (int j = 0; j < SlabRegs<KT, ACT, COHERENT, MIDL>::FR; ++j) {
+    const int f = tid + j * FT;
+    if (f < n * KT * 4) {
+      const SlabFrag F = slab_frag(f, n, nm);
+      v4u a, b = v4u{0u, 0u, 0u, 0u};
+      if constexpr (COHERENT) {
+        const uint64_t* h = r.h[j];
+        a = v4u{(uint32_t)h[0], (uint32_t)(h[0] >> 32), (uint32_t)h[1], (uint32_t)(h[1] >> 32)};
+        b = v4u{(uint32_t)h[2], (uint32_t)(h[2] >> 32), (uint32_t)h[3], (uint32_t)(h[3] >> 32)};
+      } else {
+        a = r.v0[j];
+        b = r.v1[j];
+      }
+      if constexpr (ACT == DGM_ACT_NVFP4) {
+        // -> f16 operand of op g for the four lane groups qd (K = 32 g + 8 qd .. +8): E2M1 -> f16
+        // exactly, times the E4M3 block scale (the products are exact in f16)
+        const uint32_t sc2 = r.s16[j] >> ((F.g & 1) * 16);      // byte 0: block 2 g, byte 1: 2 g + 1
         const v2h s01 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(sc2, 1.0f, false);
+        const uint32_t w[4] = {a.x, a.y, a.z, a.w};
 #pragma unroll
         for (int qd = 0; qd < 4; ++qd) {
           const _Float16 sv = qd < 2 ? s01.x : s01.y;
@@ -732,90 +677,62 @@ DGM_DEV void slab_store(S& s, const SlabRegs<KT, ACT, COHERENT, MIDL>& r) {
           const v2h h1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w[qd], 1.0f, 1) * ss;
           const v2h h2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w[qd], 1.0f, 2) * ss;
           const v2h h3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w[qd], 1.0f, 3) * ss;
-          const v4u o = {__builtin_bit_cast(uint32_t, h0), __builtin_bit_cast(uint32_t, h1),
-                         __builtin_bit_cast(uint32_t, h2), __builtin_bit_cast(uint32_t, h3)};
-          *reinterpret_cast<v4u*>(&s.bst[kt][(qd << 4) | c][gq]) = have ? o : z;
+          *reinterpret_cast<v4u*>(&s.bst[F.kt][(qd << 4) | F.c][F.g]) =
+              v4u{__builtin_bit_cast(uint32_t, h0), __builtin_bit_cast(uint32_t, h1), __builtin_bit_cast(uint32_t, h2),
+                  __builtin_bit_cast(uint32_t, h3)};
         }
-      }
-    }
-  } else {
-#pragma unroll
-  for (int j = 0; j < SlabRegs<KT, ACT, COHERENT, MIDL>::FR; ++j) {
-    const int f = tid + j * FT;
-    if (f < KT * 64) {
-      const bool have = (r.ok >> j) & 1u;
-      v4u* dst = reinterpret_cast<v4u*>(&s.bst[f >> 6][f & 63][0]);
-      if (COHERENT) {
-        const uint64_t* h = r.h[j];
-        dst[0] = have ? v4u{(uint32_t)h[0], (uint32_t)(h[0] >> 32), (uint32_t)h[1], (uint32_t)(h[1] >> 32)} : z;
-        if (ACT != DGM_ACT_MXFP4)
-          dst[S::BV - 1] = have ? v4u{(uint32_t)h[2], (uint32_t)(h[2] >> 32), (uint32_t)h[3], (uint32_t)(h[3] >> 32)} : z;
       } else {
-        dst[0] = have ? r.v0[j] : z;
-        if (ACT != DGM_ACT_MXFP4) dst[S::BV - 1] = have ? r.v1[j] : z;
+        v4u* dst = reinterpret_cast<v4u*>(&s.bst[F.kt][(F.g << 4) | F.c][0]);
+        dst[0] = a;
+        if constexpr (ACT != DGM_ACT_MXFP4) dst[S::BV - 1] = b;
       }
-    }
-  }
-  }
-  constexpr int KG = (KT + 3) / 4;
-  if constexpr (ACT == DGM_ACT_NVFP4) {
-    // (no scale plane: the scales are folded into the f16 operands)
-  } else if constexpr (ACT == DGM_ACT_QOQ) {
-#pragma unroll
-    for (int j = 0; j < SlabRegs<KT, ACT, COHERENT, MIDL>::FR; ++j) {
-      const int f = tid + j * FT;
-      if (f < KT * 64) {
-        const bool have = (r.ok >> j) & 1u;
-        const int kt = f >> 6, l = f & 63;
-        int s0, s1;
-        if (COHERENT) {
-          const uint64_t* h = r.h[j];
-          s0 = i8_sum16((uint32_t)h[0], (uint32_t)(h[0] >> 32), (uint32_t)h[1], (uint32_t)(h[1] >> 32));
-          s1 = i8_sum16((uint32_t)h[2], (uint32_t)(h[2] >> 32), (uint32_t)h[3], (uint32_t)(h[3] >> 32));
-        } else {
-          s0 = i8_sum16(r.v0[j].x, r.v0[j].y, r.v0[j].z, r.v0[j].w);
-          s1 = i8_sum16(r.v1[j].x, r.v1[j].y, r.v1[j].z, r.v1[j].w);
-        }
-        s0 = have ? s0 : 0;
-        s1 = have ? s1 : 0;
-        // (the branch is wave-uniform: a wave's 64 lanes are the 4 lane groups of one K-tile)
-        s0 += __shfl_xor(s0, 16);
-        s0 += __shfl_xor(s0, 32);
-        s1 += __shfl_xor(s1, 16);
-        s1 += __shfl_xor(s1, 32);
-        if (l < 16) {
-          if (MIDL) {            // intermediate rows (L2): the K-tile's promote coefficients
-            const float sm0 = have ? __uint_as_float((uint32_t)r.sc2[j]) : 0.f;
-            const float sm1 = have ? __uint_as_float((uint32_t)(r.sc2[j] >> 32)) : 0.f;
+      if constexpr (ACT == DGM_ACT_QOQ) {
+        // the K-tile's value sums over its four lane groups (a quad of lanes)
+        int s0 = i8_sum16(a.x, a.y, a.z, a.w), s1 = i8_sum16(b.x, b.y, b.z, b.w);
+        s0 += __builtin_amdgcn_mov_dpp(s0, 0xB1, 0xF, 0xF, false);      // quad_perm [1,0,3,2]
+        s0 += __builtin_amdgcn_mov_dpp(s0, 0x4E, 0xF, 0xF, false);      // quad_perm [2,3,0,1]
+        s1 += __builtin_amdgcn_mov_dpp(s1, 0xB1, 0xF, 0xF, false);
+        s1 += __builtin_amdgcn_mov_dpp(s1, 0x4E, 0xF, 0xF, false);
+        if (F.g == 0) {
+          if constexpr (MIDL) {    // intermediate rows (L2): the K-tile's promote coefficients
+            const float sm0 = __uint_as_float((uint32_t)r.sc2[j]), sm1 = __uint_as_float((uint32_t)(r.sc2[j] >> 32));
             const float x0 = (float)s0, x1 = (float)s1;
-            s.qc[l][kt] = make_float4(sm0, sm1 * 0.0625f, 8.f * x1 * sm1, -fmaf(x1, sm1, x0 * sm0));
-          } else {               // input rows (L1): per K-tile
-            s.xsum[l][kt] = s0 + s1;
+            s.qc[F.c][F.kt] = make_float4(sm0, sm1 * 0.0625f, 8.f * x1 * sm1, -fmaf(x1, sm1, x0 * sm0));
+          } else {                 // input rows (L1): per K-tile
+            s.xsum[F.c][F.kt] = s0 + s1;
           }
         }
       }
     }
-    if (!MIDL && tid < 16) s.xsc[tid] = (r.ok >> 8) & 1u ? r.fsc : 0.f;
-  } else if constexpr (ACT == DGM_ACT_FP8F128) {
-    // input rows with one fp32 scale per K-tile (the dword slab_load read for K-tile 4 g + j is
-    // that scale: the same row pitch as four E8M0 bytes): per (K-tile, column) to s.xf; the
-    // block-scaled op gets unit activation scales
-    if (tid < KG * 64) {
-      s.bsc[tid >> 6][tid & 63] = 0x7f7f7f7fu;
-      if ((tid & 63) < 16) {
+  }
+  constexpr int KG = (KT + 3) / 4;
+  if constexpr (ACT == DGM_ACT_QOQ) {
+    if constexpr (!MIDL) {
+      if (tid < 16) s.xsc[tid] = r.fsc;
+    }
+  } else if constexpr (ACT != DGM_ACT_NVFP4) {
+    const int u = FT - 1 - tid, c = u / KG, gs = u % KG;
+    if (c < n) {
+      if constexpr (ACT == DGM_ACT_FP8F128) {
+        // input rows with one fp32 scale per K-tile (the dwords read are those scales: the same row
+        // pitch as four E8M0 bytes per 32): per (K-tile, column) to s.xf; the block-scaled op gets
+        // unit activation scales
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int kt = 4 * (tid >> 6) + j;
-          if (kt < KT) s.xf[kt][tid & 63] = (r.ok >> (8 + j)) & 1u ? __uint_as_float(r.sb[j]) : 0.f;
+        for (int j = 0; j < 4; ++j)
+          if (4 * gs + j < KT) s.xf[4 * gs + j][c] = __uint_as_float(r.sb[j]);
+#pragma unroll
+        for (int kq = 0; kq < 4; ++kq) s.bsc[gs][(kq << 4) | c] = 0x7f7f7f7fu;
+      } else {
+        // lane group kq's dword: byte kq of each K-tile's dword (padding tiles 127)
+#pragma unroll
+        for (int kq = 0; kq < 4; ++kq) {
+          uint32_t w = 0;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) w |= ((r.sb[j] >> (8 * kq)) & 0xffu) << (8 * j);
+          s.bsc[gs][(kq << 4) | c] = w;
         }
       }
     }
-  } else if (tid < KG * 64) {
-    uint32_t w = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      w |= ((r.ok >> (8 + j)) & 1u ? (r.sb[j] >> (8 * ((tid & 63) >> 4))) & 0xffu : 127u) << (8 * j);
-    s.bsc[tid >> 6][tid & 63] = w;
   }
   if (tid < 16) s.slab_w[tid] = r.w;
 }
@@ -1100,11 +1017,14 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
     wait_mem();
     if (e0 >= 0) {
       const uint64_t m = __ballot(lane < R && s.exp_of_route[lane] == e0);
-      uint64_t mc = m;
-      for (int i = 0; i < (lane & 15); ++i) mc &= mc - 1;     // drop the first c members
-      const int rt = mc ? (int)__builtin_ctzll(mc) : 0;         // the route of slab column c
-      slab_load<KT1, ACT, FEIN, false>(pre, p.x, p.xsf, XB, (int)__popcll(m), [rt, tkm](int) { return div_small(rt, tkm); },
-                                       [rt](int) { return s.route_w[rt]; });
+      auto route_of = [m](int c) {                              // the route of slab column c
+        uint64_t mc = m;
+        for (int i = 0; i < c; ++i) mc &= mc - 1;               // drop the first c members
+        return (int)__builtin_ctzll(mc);
+      };
+      slab_load<KT1, ACT, FEIN, false>(pre, p.x, p.xsf, XB, (int)__popcll(m),
+                                       [route_of, tkm](int c) { return div_small(route_of(c), tkm); },
+                                       [route_of](int c) { return s.route_w[route_of(c)]; });
       const size_t blk = l1_blk(e0, (int)blockIdx.x % QN1);
       load_scales_blk(blk, sd);
       const uint8_t* b = p.w1v + blk * KT1 * 1024 + lane * 16;
@@ -1909,13 +1829,8 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
           if (tid == 0 && !seen) st[3] = wall_clock();
           seen = true;
         }
-        if constexpr (ACT == DGM_ACT_QOQ || ACT == DGM_ACT_NVFP4) {
-          load_slab(pre, a, s0);            // (pre holds nothing between items)
-          slab_store(s, pre);
-        } else {
-          const int rb = r0 + s0;
-          stage_slab<KT2, ACT2, !BIG>(s, p.mid, p.mid_sf, MB, n - s0, [rb](int cc) { return rb + cc; });
-        }
+        load_slab(pre, a, s0);              // (pre holds nothing between items)
+        slab_store(s, pre);
         staged = key;
         __syncthreads();
       }
