@@ -511,24 +511,24 @@ def _moe_args(y, l1, l2, b, stats, activation_clamp, num_tokens=None, phase_stam
     assert m <= b.num_max_tokens_per_rank
     E_l, H, I = b.num_local_experts, b.hidden, b.intermediate_hidden
     kg = lambda k: (k // 128 + 3) // 4
-    assert tuple(w1.shape) == (E_l, 2 * I // 16, H // 128, 64, 16) and w1.dtype == torch.uint8, w1.shape
-    assert tuple(w2.shape) == (E_l, H // 16, I // 128, 64, 16) and w2.dtype == torch.uint8, w2.shape
+    assert w1.shape == (E_l, 2 * I // 16, H // 128, 64, 16) and w1.dtype == torch.uint8, w1.shape
+    assert w2.shape == (E_l, H // 16, I // 128, 64, 16) and w2.dtype == torch.uint8, w2.shape
     if nv:    # E4M3 scales [E, N/16, K/128, 2, 16, 4]
-        assert tuple(sf1.shape) == (E_l, 2 * I // 16, H // 128, 2, 16, 4) and sf1.dtype == torch.uint8, sf1.shape
-        assert tuple(sf2.shape) == (E_l, H // 16, I // 128, 2, 16, 4) and sf2.dtype == torch.uint8, sf2.shape
+        assert sf1.shape == (E_l, 2 * I // 16, H // 128, 2, 16, 4) and sf1.dtype == torch.uint8, sf1.shape
+        assert sf2.shape == (E_l, H // 16, I // 128, 2, 16, 4) and sf2.dtype == torch.uint8, sf2.shape
         for g in global_scales:
             if g is not None:
                 _lib.require_gpu(g)
                 assert g.dtype == torch.float32 and g.numel() == E_l and g.is_contiguous()
     elif qoq:   # meta [E, N/16, K/128, 16] (z | s2 << 4 per row), row scales s1 [E, N]
         _lib.require_gpu(rs1, rs2)
-        assert tuple(sf1.shape) == (E_l, 2 * I // 16, H // 128, 16) and sf1.dtype == torch.uint8, sf1.shape
-        assert tuple(sf2.shape) == (E_l, H // 16, I // 128, 16) and sf2.dtype == torch.uint8, sf2.shape
-        assert tuple(rs1.shape) == (E_l, 2 * I) and rs1.dtype == torch.float32 and rs1.is_contiguous(), rs1.shape
-        assert tuple(rs2.shape) == (E_l, H) and rs2.dtype == torch.float32 and rs2.is_contiguous(), rs2.shape
+        assert sf1.shape == (E_l, 2 * I // 16, H // 128, 16) and sf1.dtype == torch.uint8, sf1.shape
+        assert sf2.shape == (E_l, H // 16, I // 128, 16) and sf2.dtype == torch.uint8, sf2.shape
+        assert rs1.shape == (E_l, 2 * I) and rs1.dtype == torch.float32 and rs1.is_contiguous(), rs1.shape
+        assert rs2.shape == (E_l, H) and rs2.dtype == torch.float32 and rs2.is_contiguous(), rs2.shape
     else:
-        assert tuple(sf1.shape) == (E_l, 2 * I // 16, kg(H), 64, 4) and sf1.dtype == torch.uint8, sf1.shape
-        assert tuple(sf2.shape) == (E_l, H // 16, kg(I), 64, 4) and sf2.dtype == torch.uint8, sf2.shape
+        assert sf1.shape == (E_l, 2 * I // 16, kg(H), 64, 4) and sf1.dtype == torch.uint8, sf1.shape
+        assert sf2.shape == (E_l, H // 16, kg(I), 64, 4) and sf2.dtype == torch.uint8, sf2.shape
     assert all(t.is_contiguous() for t in (w1, sf1, w2, sf2))
     if stats is not None:
         assert stats.dtype == torch.int32 and stats.numel() == E_l
@@ -544,27 +544,37 @@ def _moe_args(y, l1, l2, b, stats, activation_clamp, num_tokens=None, phase_stam
         assert fe_keys.dtype in (torch.int32, torch.uint32) and fe_keys.is_contiguous(), fe_keys.dtype
         assert fe_keys.numel() >= m * b.num_experts, (fe_keys.numel(), m, b.num_experts)
         sel = (sel[0] & _lib.FE_FORCE_BALANCED if sel else 0, sel[1] if sel else 0)
+    # (the fields of options that are off stay at their zero: each one set costs time on a call that
+    # the GPU finishes in 25 us)
     args = _lib.MoeArgs(num_tokens=m, hidden=b.hidden, intermediate=b.intermediate_hidden,
                         num_experts=b.num_experts, expert_begin=b.expert_begin, num_local_experts=E_l,
                         topk=b.num_topk, act_format=_lib.ACT_FORMATS[act],
                         activation_clamp=float(activation_clamp if activation_clamp is not None else 3.0e38),
-                        fast_math=int(bool(fast_math)), select_in_mega=int(sel is not None),
-                        fe_flags=sel[0] if sel else 0, token_offset=sel[1] if sel else 0,
+                        fast_math=int(bool(fast_math)),
                         w1_values=w1.data_ptr(), w1_scales=sf1.data_ptr(), w2_values=w2.data_ptr(),
-                        w2_scales=sf2.data_ptr(), recv_stats=stats.data_ptr() if stats is not None else None,
-                        y=y.data_ptr(), buffer=b.buffer.data_ptr(), layout=ctypes.pointer(b.layout),
-                        phase_stamps=phase_stamps.data_ptr() if phase_stamps is not None else None,
-                        phase_stamp_rows=phase_stamps.numel() // 8 if phase_stamps is not None else 0,
-                        w1_row_scales=rs1.data_ptr() if qoq else None,
-                        w2_row_scales=rs2.data_ptr() if qoq else None,
-                        l1_global_scales=global_scales[0].data_ptr() if global_scales[0] is not None else None,
-                        l2_global_scales=global_scales[1].data_ptr() if global_scales[1] is not None else None,
-                        fe_in_mega=int(fe is not None),
-                        hidden_states=fe[0].data_ptr() if fe is not None else None,
-                        router_weight=fe[1].data_ptr() if fe is not None else None,
-                        fe_keys=fe_keys.data_ptr() if fe_keys is not None else None,
-                        host_error=b._host_err_dev, debug_flags=getattr(b, "_debug_flags", 0),
-                        launch_flags=_lib.LAUNCH_COOPERATIVE if cooperative_launch(b) else 0)
+                        w2_scales=sf2.data_ptr(), y=y.data_ptr(), buffer=b.buffer.data_ptr(),
+                        layout=ctypes.pointer(b.layout), host_error=b._host_err_dev)
+    if sel is not None:
+        args.select_in_mega, args.fe_flags, args.token_offset = 1, sel[0], sel[1]
+    if stats is not None:
+        args.recv_stats = stats.data_ptr()
+    if qoq:
+        args.w1_row_scales, args.w2_row_scales = rs1.data_ptr(), rs2.data_ptr()
+    if global_scales[0] is not None:
+        args.l1_global_scales = global_scales[0].data_ptr()
+    if global_scales[1] is not None:
+        args.l2_global_scales = global_scales[1].data_ptr()
+    if fe is not None:
+        args.fe_in_mega, args.hidden_states, args.router_weight = 1, fe[0].data_ptr(), fe[1].data_ptr()
+    if fe_keys is not None:
+        args.fe_keys = fe_keys.data_ptr()
+    if phase_stamps is not None:
+        args.phase_stamps, args.phase_stamp_rows = phase_stamps.data_ptr(), phase_stamps.numel() // 8
+    debug = getattr(b, "_debug_flags", 0)
+    if debug:
+        args.debug_flags = debug
+    if cooperative_launch(b):
+        args.launch_flags = _lib.LAUNCH_COOPERATIVE
     if phase_stamps is not None:
         assert phase_stamps.dtype == torch.int64 and phase_stamps.is_cuda and phase_stamps.is_contiguous()
     return args
