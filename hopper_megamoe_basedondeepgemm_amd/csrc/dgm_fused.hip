@@ -1320,13 +1320,8 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
                            : !has_next ? (hand ? reinterpret_cast<const uint8_t*>(p.w2s) + l2_blk(v0) * KT2 * 128 + slane : sdummy)
                                        : nq == q0 ? csb : stile_base(nq);
       const uint8_t* nsbd = hand ? sdummy : nsb;
-      // (MXFP, QoQ: the next item's scale and slab loads are issued in the K loop, after the
-      // tile loads of its first KT1 - KR ops, so that the loop starts as soon as its first tile
-      // is in)
-      if constexpr (ACT == DGM_ACT_NVFP4) {
-        if (has_next && nq != q0) load_scales(nq, sn);
-        if (restage) load_slab(pre, na, ns0);
-      }
+      // (the next item's scale and slab loads are issued in the K loop, after the tile loads of its
+      // first KT1 - KR ops, so that the loop starts as soon as its first tile is in)
       const float wt_r = s.slab_w[c];
       const float sx = ACT == DGM_ACT_QOQ ? s.xsc[c] : 1.f;       // QoQ: the token's activation scale
       // the unit after q1, claimed during the item that finishes q0 (after its loads; the value
@@ -1423,6 +1418,9 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
           } else {
             wr[t % KR] = ld_stream_after(t + KR - KT1 < KT2 ? nb : nbd, (t + KR - KT1) * 1024, acc);
             sr[t % KR] = ld_stream32_after(t + KR - KT1 < KT2 ? nsb : nsbd, (t + KR - KT1) * 128, acc);
+          }
+          if constexpr (t == KT1 - KR) {
+            if (restage) load_slab(pre, na, ns0);
           }
         });
       } else if constexpr (F128) {
