@@ -211,8 +211,16 @@ struct FusedSmem {
       int eoff[ML];
       int wcnt[BIG ? NW : 1][BIG ? ML : 1];   // (BIG) routes per wave and expert
     };
-    U4 bst[KTM][64][BV];               // B slab in matrix-core fragment order
+    U4 bst[KTM * BV * 64];             // B slab in matrix-core fragment order: frag()
   };
+  // The j-th 16-byte piece of lane l's operand of K-tile t. The pieces are in planes, so a wave's read
+  // of one is 1 KB contiguous: with a lane's pieces side by side (64 bytes for NVFP4) each read met
+  // four-way bank conflicts, and the eight waves' reads took longer than their weight tiles (NVFP4,
+  // 64 tokens: K loop of an L1 unit 6.3 -> 4.7 us, whole call 324 -> 321 us; A-MXFP8, 512 tokens
+  // 446 -> 442). FP8F128 keeps the pieces side by side: the planes cost it four spilled registers
+  // (5 tokens 54.9 -> 55.5 us).
+  static constexpr bool PLANES = ACT != DGM_ACT_FP8F128;
+  static DGM_DEV int frag(int t, int j, int l) { return PLANES ? (t * BV + j) * 64 + l : (t * 64 + l) * BV + j; }
   uint32_t bsc[(KTM + 3) / 4][64];     // its E8M0 scales, 4 K-tiles per dword
   // QoQ slab extras. Input rows (L1): per column and K-tile the sum of the column's int8
   // values (for the zero-point term) and per column the token's scale. Intermediate rows (L2):
@@ -677,14 +685,13 @@ DGM_DEV void slab_store(S& s, const SlabRegs<KT, ACT, COHERENT, MIDL>& r) {
           const v2h h1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w[qd], 1.0f, 1) * ss;
           const v2h h2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w[qd], 1.0f, 2) * ss;
           const v2h h3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w[qd], 1.0f, 3) * ss;
-          *reinterpret_cast<v4u*>(&s.bst[F.kt][(qd << 4) | F.c][F.g]) =
+          *reinterpret_cast<v4u*>(&s.bst[S::frag(F.kt, F.g, (qd << 4) | F.c)]) =
               v4u{__builtin_bit_cast(uint32_t, h0), __builtin_bit_cast(uint32_t, h1), __builtin_bit_cast(uint32_t, h2),
                   __builtin_bit_cast(uint32_t, h3)};
         }
       } else {
-        v4u* dst = reinterpret_cast<v4u*>(&s.bst[F.kt][(F.g << 4) | F.c][0]);
-        dst[0] = a;
-        if constexpr (ACT != DGM_ACT_MXFP4) dst[S::BV - 1] = b;
+        *reinterpret_cast<v4u*>(&s.bst[S::frag(F.kt, 0, (F.g << 4) | F.c)]) = a;
+        if constexpr (ACT != DGM_ACT_MXFP4) *reinterpret_cast<v4u*>(&s.bst[S::frag(F.kt, S::BV - 1, (F.g << 4) | F.c)]) = b;
       }
       if constexpr (ACT == DGM_ACT_QOQ) {
         // the K-tile's value sums over its four lane groups (a quad of lanes)
@@ -933,7 +940,7 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
     // top-k from the frontend's keys, as the frontend would have done: the keys of TC tokens at
     // a time go through LDS (the slab area, unused until the L1 phase; one coalesced pass),
     // then one wave selects per token
-    uint32_t* lg = reinterpret_cast<uint32_t*>(&s.bst[0][0][0]);
+    uint32_t* lg = reinterpret_cast<uint32_t*>(&s.bst[0]);
     const int TC = (int)(sizeof(s.bst) / 4) / p.E;
     for (int t0 = 0; t0 < p.M; t0 += TC) {
       const int tn = p.M - t0 < TC ? p.M - t0 : TC;
@@ -1283,7 +1290,8 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
     // the previous item's epilogue, before its stores: read at the loop's top, they could land
     // in registers of those stores and wait for them (and so for the whole ring).
     auto bfrag = [lane](int t) __attribute__((always_inline)) {
-      return ACT == DGM_ACT_MXFP4 ? as_v8i(s.bst[t][lane][0]) : as_v8i(s.bst[t][lane][0], s.bst[t][lane][Smem::BV - 1]);
+      return ACT == DGM_ACT_MXFP4 ? as_v8i(s.bst[Smem::frag(t, 0, lane)])
+                                   : as_v8i(s.bst[Smem::frag(t, 0, lane)], s.bst[Smem::frag(t, Smem::BV - 1, lane)]);
     };
     v8i bq0 = {}, bq1 = {};
     uint32_t bs0 = 0;
@@ -1400,7 +1408,7 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
         // f16 in LDS (read one tile ahead); scale dwords stream in their own ring
         U4 bn[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) bn[j] = s.bst[0][lane][j];
+        for (int j = 0; j < 4; ++j) bn[j] = s.bst[Smem::frag(0, j, lane)];
         static_for<KT1>([&](auto tc) {
           constexpr int t = decltype(tc)::value;
           if constexpr (t == CT) claim_ahead();
@@ -1409,7 +1417,7 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
           for (int j = 0; j < 4; ++j) bc[j] = bn[j];
           if constexpr (t + 1 < KT1) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) bn[j] = s.bst[t + 1][lane][j];
+            for (int j = 0; j < 4; ++j) bn[j] = s.bst[Smem::frag(t + 1, j, lane)];
           }
           acc = nvfp4_tile(wr[t % KR], sr[t % KR], bc, acc);
           if constexpr (t + KR < KT1) {
@@ -1883,7 +1891,8 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
 #pragma unroll
       for (int j = 0; j < RB; ++j) acc[j] = v4f{0.f, 0.f, 0.f, 0.f};
       auto bfrag = [lane](int k) __attribute__((always_inline)) {
-        return ACT == DGM_ACT_MXFP4 ? as_v8i(s.bst[k][lane][0]) : as_v8i(s.bst[k][lane][0], s.bst[k][lane][Smem::BV - 1]);
+        return ACT == DGM_ACT_MXFP4 ? as_v8i(s.bst[Smem::frag(k, 0, lane)])
+                                     : as_v8i(s.bst[Smem::frag(k, 0, lane)], s.bst[Smem::frag(k, Smem::BV - 1, lane)]);
       };
       v8i bq0 = bfrag(0), bq1 = bfrag(1 % KT2);
       if constexpr (ACT == DGM_ACT_QOQ) {
@@ -1948,7 +1957,7 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
       } else if constexpr (ACT == DGM_ACT_NVFP4) {
         U4 bn[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) bn[j] = s.bst[0][lane][j];
+        for (int j = 0; j < 4; ++j) bn[j] = s.bst[Smem::frag(0, j, lane)];
         static_for<TI>([&](auto tc) {
           constexpr int t = decltype(tc)::value;
           if constexpr (t == CT) claim_ahead();
@@ -1958,7 +1967,7 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
           for (int i = 0; i < 4; ++i) bc[i] = bn[i];
           if constexpr (t + 1 < TI) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) bn[i] = s.bst[(t + 1) % KT2][lane][i];
+            for (int i = 0; i < 4; ++i) bn[i] = s.bst[Smem::frag((t + 1) % KT2, i, lane)];
           }
           acc[j] = nvfp4_tile(wr[k], sr[k], bc, acc[j]);
           if constexpr (t + KT2 < TI) {
