@@ -293,11 +293,11 @@ __global__ void __launch_bounds__(256) k_quantize_nvfp4(const void* __restrict__
 // ------------------------------------------------------------------ QoQ W4A8 packer
 // One wave per weight row: row amax -> s1 (bf16), then sixteen lanes per K128 group, eight elements
 // each (a wave covers 512 elements of the row per step).
-// plane != null: the split path's int4 form (s2 clamped to 127 instead of 15, which |w8| <= 112
-// never reaches; s2 | z << 8 | bf16(s1) << 16 per (row, K128 group) instead of s2o / zo / s1o)
+// plane != null: the split path's int4 form (its clamp of s2 at 127 instead of 15 never applies:
+// |w8| <= 112; s2 | z << 8 | bf16(s1) << 16 per (row, K128 group) instead of s2o / zo / s1o)
 // NJ > 0: the row (K <= 512 NJ, 16-byte aligned) is read once and held in registers; NJ = 0: any row,
 // element loads, read once per pass. (A lane per group, with element loads and three passes, took
-// 254 us for 63 M bf16 elements of K = 3072 and for 31 M of K = 1280; this takes 45 and 27 us, bound by
+// 254 us for 63 M bf16 elements of K = 3072 and for 31 M of K = 1280; this takes 40 and 24 us, bound by
 // about twenty VALU operations per element.)
 template <int SRC, int NJ>
 __global__ void __launch_bounds__(256) k_quantize_qoq(const void* __restrict__ w, int64_t rows, int K,
@@ -364,9 +364,14 @@ __global__ void __launch_bounds__(256) k_quantize_qoq(const void* __restrict__ w
     }
     mx = max_lanes16(mx);
     mn = -max_lanes16(-mn);
-    const float s2 = fminf(fmaxf(ceilf((mx - mn) / 15.0f), 1.f), plane ? 127.f : 15.f);
-    const float z = fminf(fmaxf(rintf(-mn / s2), 0.f), 15.f);
-    const float r2 = 1.0f / s2;
+    // s2 = ceil((mx - mn) / 15) of integers up to 224 (the quotient is an integer or at least 1/15
+    // above one), at most 15; its reciprocal from the hardware's with one Newton step, correctly
+    // rounded for these (Markstein, as above)
+    const float s2 = fmaxf(ceilf(fmaf(mx - mn, 1.0f / 15.0f, -0.01f)), 1.f);
+    float r2 = __builtin_amdgcn_rcpf(s2);
+    r2 = fmaf(fmaf(-s2, r2, 1.0f), r2, r2);
+    float z = -mn * r2;
+    z = __builtin_amdgcn_fmed3f(rintf(fmaf(fmaf(-z, s2, -mn), r2, z)), 0.f, 15.f);
     uint32_t n[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
