@@ -402,7 +402,9 @@ DGM_DEV void big_dispatch(S& s, const int64_t* __restrict__ topk_idx, const floa
       w[k] = topk_w[r];
     }
   }
-  for (int i = tid; i < NW * S::ML; i += FT) (&s.wcnt[0][0])[i] = 0;
+#pragma unroll
+  for (int v = 0; v < NW; ++v)
+    for (int x = tid; x < E_local; x += FT) s.wcnt[v][x] = 0;
   __syncthreads();
   int e[STEPS], pos[STEPS];
 #pragma unroll
