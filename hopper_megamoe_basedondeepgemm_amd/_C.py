@@ -88,7 +88,7 @@ def _run_fused(act, y, l1, l2, stats, s1, s2, buffer, ptrs, rank, max_tokens, nu
     w1 = (l1[0], l1[1], s1)
     w2 = (l2[0], l2[1], s2)
     # one launch of the persistent kernel (beyond its limits, 1024 routes, 256 tokens, 512 local
-    # experts, the E4M3 layer runs as the split path's kernels, with the same results)
+    # experts, the E4M3 layer runs as the split path's launches, with the same results)
     mega._fused(y, w1, w2, b, stats, clamp, phase_stamps=phase_stamps, fast_math=fast_math, fmt=act,
                 fe_keys=fe_keys, act=act)
 

@@ -26,6 +26,10 @@
 // asc). Workgroup 0 also publishes the routing and the pool, the recv stats and the zero rows
 // of tokens without a local route.
 //
+// Launches. One launch runs the whole layer, or (the split calls, and the large-batch form) one
+// launch runs L1 and one L2 without the combine, which is then a kernel of its own: no workgroup of
+// those waits on another.
+//
 // Hand-offs between workgroups go through HBM with agent-coherent accesses only: the data
 // (intermediate codes and scales, bf16 route outputs) is written with relaxed agent-scope
 // atomic stores (write-through, "sc1") and read with agent-scope atomic loads, and the
@@ -772,10 +776,10 @@ DGM_DEV long long wall_clock() { return (long long)__builtin_amdgcn_s_memrealtim
 // dispatch. It runs one phase per launch (L1, or L2 without the combine, which is a launch of its
 // own) and so has no wait on another workgroup: calls beyond the plain form's limits never needed
 // the whole grid resident, and two of them on two streams must not wait for each other's CUs.
-// E384 H3072 I1280, 512 tokens, whole call: A-MXFP8 456 us (259 L1, 151 L2; 1.71 + 0.89 GB read,
-// 6.6 and 5.9 TB/s), one of eight ranks' experts, A-MXFP4, 106 us. The kernels it replaced (a
-// one-workgroup dispatch, L1 and L2 that load an item's weights before its first op) took 1227 and
-// 367 us with the VALU router. Bound by the weight stream and, in L2, the items' fixed cost.
+// E384 H3072 I1280, 512 tokens, whole call: A-MXFP8 442 us (259 L1, 151 L2 when first measured, at
+// 456; 1.71 + 0.89 GB read, 6.6 and 5.9 TB/s), one of eight ranks' experts, A-MXFP4, 101 us. The
+// kernels it replaced (a one-workgroup dispatch, L1 and L2 that load an item's weights before its
+// first op) took 1227 and 367 us, with the VALU router. Bound by the weight stream and, in L2, the items' fixed cost.
 // Measured and not taken: the whole layer in one launch (455 / 101 us, but with the waits), runs of
 // consecutive units per claim, whose slab is staged once (+4 %: the runs' uneven end).
 constexpr int FORM_PLAIN = 0, FORM_FEIN = 1, FORM_EARLY = 2, FORM_TAIL = 3, FORM_BIG = 4;

@@ -767,7 +767,7 @@ def fused_last_form(b):
 
 
 def mxfp4_mega_moe_split(y, l1_weights, l2_weights, sym_buffer, *args, **kwargs):
-    """deep_gemm/mega/__init__.py:579 split API: the same layer as separate launches (dispatch,
+    """deep_gemm/mega/__init__.py:579 split API: the same layer as separate launches (dispatch +
     L1 + SwiGLU + requant, L2, combine) with the fused path's numerics, on an "mxfp4" / "mxfp8"
     fused buffer. Arguments as ``mxfp4_mega_moe`` (:340; activation_clamp default None = no
     clamp)."""

@@ -339,9 +339,10 @@ int dgm_megamoe_fused_launch_noalloc(const DgmMoeArgs* args, hipStream_t stream)
 
 /* Replaces csrc/apis/mega.hpp:550 _C.mxfp4_mega_moe_split / deep_gemm/mega/__init__.py:579
  * mxfp4_mega_moe_split and :584 qoq_mega_moe_split: the same layer as separate launches instead
- * of one persistent kernel, identical numerics. MXFP4 / MXFP8: dispatch, L1, L2, combine
- * kernels; QoQ / NVFP4: the persistent kernel twice, dispatch + L1 then L2 + combine (the
- * fused kernel's limits on tokens, routes and local experts apply). fe_in_mega is rejected. */
+ * of one, identical numerics: the persistent kernel twice. MXFP4 / MXFP8 / FP8F128: dispatch + L1,
+ * then L2, then a combine launch (none waits on another workgroup); QoQ / NVFP4: dispatch + L1,
+ * then L2 + combine (the fused launch's limits on tokens, routes and local experts apply).
+ * fe_in_mega is rejected. */
 int dgm_megamoe_split_launch(const DgmMoeArgs* args, hipStream_t stream);
 
 /* Device address of pinned host memory (hipHostGetDevicePointer), e.g. for
@@ -351,8 +352,8 @@ int dgm_host_device_pointer(const void* host, void** device);
 /* Diagnostics (no counterpart in the reference). dgm_device_cu_count: compute units of the
  * current device. dgm_fused_workgroups: workgroups of the persistent kernel for a shape (0 before
  * its first launch). dgm_fused_last_form: the form its last launch for a shape ran, 0 plain,
- * 1 with the in-kernel frontend, 2 with early weight streaming, 3 with tail half units (-1
- * before its first launch).
+ * 1 with the in-kernel frontend, 2 with early weight streaming, 3 with tail half units, 4 large
+ * batch (-1 before its first launch).
  * The lane-layout probes of the tests live in a library of their own (include/dgm_probe.h). */
 int dgm_device_cu_count(void);
 int dgm_fused_workgroups(int hidden, int intermediate, int act_format);
