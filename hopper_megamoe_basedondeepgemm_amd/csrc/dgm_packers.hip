@@ -297,8 +297,8 @@ __global__ void __launch_bounds__(256) k_quantize_nvfp4(const void* __restrict__
 // |w8| <= 112; s2 | z << 8 | bf16(s1) << 16 per (row, K128 group) instead of s2o / zo / s1o)
 // NJ > 0: the row (K <= 512 NJ, 16-byte aligned) is read once and held in registers; NJ = 0: any row,
 // element loads, read once per pass. (A lane per group, with element loads and three passes, took
-// 254 us for 63 M bf16 elements of K = 3072 and for 31 M of K = 1280; this takes 40 and 24 us, bound by
-// about twenty VALU operations per element.)
+// 254 us for 63 M bf16 elements of K = 3072 and for 31 M of K = 1280; this takes 35 and 22 us, bound by
+// about sixteen VALU operations per element: 40 and 24 us with a corrected quotient for every code.)
 template <int SRC, int NJ>
 __global__ void __launch_bounds__(256) k_quantize_qoq(const void* __restrict__ w, int64_t rows, int K,
                                                       uint8_t* __restrict__ packed, uint8_t* __restrict__ s2o,
@@ -336,11 +336,12 @@ __global__ void __launch_bounds__(256) k_quantize_qoq(const void* __restrict__ w
   for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
   const float s1 = round_bf16(fmaxf(amax / 120.0f, 1e-30f));
   if (lane == 0 && !plane) s1o[row] = s1;
-  // Quotients by s1 (and by s2, an integer <= 127) as a product with the correctly rounded
-  // reciprocal and one fma correction of its remainder: the correctly rounded quotient (Markstein
-  // 1990), for divisors and quotients far from the ends of the exponent range and a divisor whose
-  // mantissa is not all ones (s1 has eight bits). Rows with s1 outside it (an infinite or huge
-  // element) divide.
+  // rint(v / s1), |v / s1| <= 121. bf16 / fp16 sources: the product with the correctly rounded
+  // reciprocal, added to 384, so that the one rounding is to a multiple of 2^-15: a quotient on a
+  // half integer (off by at most 2^-17 in the product) lands on it, and any other, at least 2^-13
+  // away from one (eleven bits over eight), stays on its side. fp32 sources: the correctly rounded
+  // quotient, the product corrected by its remainder (Markstein 1990; the divisor, of eight bits, has no
+  // mantissa of all ones). Rows with s1 outside the range (an infinite or huge element) divide.
   const bool fast = __builtin_amdgcn_readfirstlane(s1 >= 0x1p-100f && s1 <= 0x1p100f) != 0;     // (one s1 per wave)
   const float r1 = 1.0f / s1;
   const int G = K / 128;
@@ -349,8 +350,12 @@ __global__ void __launch_bounds__(256) k_quantize_qoq(const void* __restrict__ w
     if (fast) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const float t = v[i] * r1;
-        q[i] = fmaf(fmaf(-t, s1, v[i]), r1, t);
+        if constexpr (SRC != SRC_F32) {
+          q[i] = fmaf(v[i], r1, 384.f) - 384.f;
+        } else {
+          const float t = v[i] * r1;
+          q[i] = fmaf(fmaf(-t, s1, v[i]), r1, t);
+        }
       }
     } else {
 #pragma unroll
@@ -372,14 +377,19 @@ __global__ void __launch_bounds__(256) k_quantize_qoq(const void* __restrict__ w
     r2 = fmaf(fmaf(-s2, r2, 1.0f), r2, r2);
     float z = -mn * r2;
     z = __builtin_amdgcn_fmed3f(rintf(fmaf(fmaf(-z, s2, -mn), r2, z)), 0.f, 15.f);
-    uint32_t n[8];
+    // rint(q / s2 + z) in 0 .. 15, as the last bits of 2^23 + code: the sum with 2048 rounds to a
+    // multiple of 2^-13 or 2^-12 (half integers land on themselves, as above; others are 1/30 away), the
+    // one with 2^23 to an integer (half to even). Marlin order from the top nibble down; the exponent
+    // bits left over add up to a constant.
+    const float zb = z + 2048.f;
+    uint32_t n[8], word;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      float t = q[i] * r2;
-      t = fmaf(fmaf(-t, s2, q[i]), r2, t);
-      n[i] = (uint32_t)__builtin_amdgcn_fmed3f(rintf(t + z), 0.f, 15.f);
-    }
-    reinterpret_cast<uint32_t*>(packed + row * (K / 2))[64 * j + lane] = marlin8(n);
+    for (int i = 0; i < 8; ++i)
+      n[i] = __float_as_uint(__builtin_amdgcn_fmed3f(fmaf(q[i], r2, zb) + (0x1p23f - 2048.f), 0x1p23f, 0x1p23f + 15.f));
+    word = n[3];
+#pragma unroll
+    for (int i = 6; i >= 0; --i) word = (word << 4) + n[i & 1 ? (i >> 1) : (i >> 1) + 4];
+    reinterpret_cast<uint32_t*>(packed + row * (K / 2))[64 * j + lane] = word - 0xFB000000u;
     if ((lane & 15) == 0) {
       const int64_t g = row * G + 4 * j + (lane >> 4);
       if (plane) {
