@@ -221,6 +221,18 @@ __global__ void k_combine(const uint16_t* __restrict__ partials, int part_rows, 
   *reinterpret_cast<uint2*>(y + (size_t)t * H + n) = make_uint2(lo, hi);
 }
 
+// The counters as an L1 launch needs them, whatever the buffer held: the set that it will use (the
+// parity word's; the launch itself clears the other one for the L2 launch) with no unit claimed and no
+// workgroup counted. Without it a claim counter left over would pass units over, and a launch that waits
+// for no arrival reports nothing.
+__global__ void __launch_bounds__(64) k_open_counters(int* __restrict__ counters) {
+  int* set = counters + CNT_SET0 + (counters[CNT_PARITY] & 1) * CNT_SET;
+  if (threadIdx.x == 0) {
+    set[CNT_STARTED] = 0;
+    set[CNT_CLAIM] = 0;
+  }
+}
+
 int g_cu_count = 0;
 
 int cu_count() {
@@ -666,8 +678,11 @@ int dgm_megamoe_split_launch(const DgmMoeArgs* A, hipStream_t stream) {
   if (A->num_tokens == 0) return 0;
   // the persistent kernel twice (dispatch + L1, then L2), then the combine: no launch has a wait
   // on another workgroup, so none needs its grid resident at once (E384, 257 tokens, FP8F128:
-  // 389 us; with the launches this replaced, see FORM_BIG, 989 us)
-  int st = fused_launch_phases(A, 1, stream);
+  // 389 us; with the launches this replaced, see FORM_BIG, 989 us). These calls keep nothing in the
+  // buffer from one to the next, the counters included
+  hipLaunchKernelGGL(k_open_counters, dim3(1), dim3(64), 0, stream, (int*)((uint8_t*)A->buffer + L->counters));
+  int st = dgm_last_launch_status();
+  if (!st) st = fused_launch_phases(A, 1, stream);
   if (!st) st = fused_launch_phases(A, 2 | 4, stream);
   return st ? st : launch_combine(A, (uint8_t*)A->buffer, L, stream);
 }

@@ -188,7 +188,11 @@ typedef struct DgmBufferLayout {
   size_t pool;                                  /* dispatch table (see DgmPoolTable)       */
   size_t mid, mid_sf;                           /* L1 -> L2 activations (pool-row order)   */
   size_t partials;                              /* bf16 [topk, max_tokens, H] route outputs (combine_partials) */
-  size_t counters;                              /* int32 scratch counters                  */
+  size_t counters;                              /* int32 counters (up to total_bytes): zero before the first
+                                                   launch, then left to the launches. The MXFP4 / MXFP8 /
+                                                   FP8F128 calls that run as several launches (split, and
+                                                   beyond 1024 routes, 256 tokens or 512 local experts)
+                                                   take them in any state */
   int32_t x_row_bytes, mid_row_bytes, max_routes, max_tokens;
   /* the shape the buffer was laid out for: every launch on it is refused (DGM_ERR_INVALID_ARGUMENT,
      before anything is enqueued) unless num_tokens <= max_tokens, topk <= topk, num_experts <=
@@ -339,8 +343,8 @@ int dgm_megamoe_fused_launch_noalloc(const DgmMoeArgs* args, hipStream_t stream)
 
 /* Replaces csrc/apis/mega.hpp:550 _C.mxfp4_mega_moe_split / deep_gemm/mega/__init__.py:579
  * mxfp4_mega_moe_split and :584 qoq_mega_moe_split: the same layer as separate launches instead
- * of one, identical numerics: the persistent kernel twice. MXFP4 / MXFP8 / FP8F128: dispatch + L1,
- * then L2, then a combine launch (none waits on another workgroup); QoQ / NVFP4: dispatch + L1,
+ * of one, identical numerics: the persistent kernel twice. MXFP4 / MXFP8 / FP8F128: the counters
+ * opened, dispatch + L1, then L2, then a combine launch (none waits on another workgroup); QoQ / NVFP4: dispatch + L1,
  * then L2 + combine (the fused launch's limits on tokens, routes and local experts apply).
  * fe_in_mega is rejected. */
 int dgm_megamoe_split_launch(const DgmMoeArgs* args, hipStream_t stream);
