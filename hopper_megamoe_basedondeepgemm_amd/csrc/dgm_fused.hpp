@@ -87,6 +87,11 @@ struct FusedParams {
                             // bit 4: tail half units
 };
 
+// Whether workgroups of a launch wait on each other (the in-kernel frontend's grid-wide arrival, L2's
+// wait for L1 units, the combine's for L2 units) and so must all be resident at once: not L1 alone,
+// and not L2 without the combine.
+constexpr bool fused_launch_waits(int phases, bool fe_in) { return fe_in || (phases & 6) == 2; }
+
 // cooperative: hipLaunchCooperativeKernel (co-residency guaranteed) instead of a plain launch
 int launch_fused(const FusedParams& prm, int hidden, int intermediate, int act, hipStream_t stream,
                  bool cooperative = false);

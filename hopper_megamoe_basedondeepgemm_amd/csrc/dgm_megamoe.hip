@@ -638,8 +638,10 @@ int dgm_fused_launch_ws(const DgmMoeArgs* A, int phases, const DgmWorkspace& w, 
     p.stamp_rows = A->phase_stamps && !(A->debug_flags & 2) ? A->phase_stamp_rows : 0;
     p.phases = phases;
     p.debug = (int16_t)(A->debug_flags & 31);
+    // (a cooperative launch costs 14-19 us of its own: only where there is something to wait for. Both
+    // launches of a split call made cooperatively: E384, 2 tokens A-MXFP8 70 us, plainly 34)
     return launch_fused(p, A->hidden, A->intermediate, A->act_format, stream,
-                        (A->launch_flags & DGM_LAUNCH_COOPERATIVE) != 0);
+                        (A->launch_flags & DGM_LAUNCH_COOPERATIVE) && fused_launch_waits(phases, A->fe_in_mega != 0));
   }
 }
 

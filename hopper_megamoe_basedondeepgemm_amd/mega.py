@@ -482,8 +482,9 @@ def cooperative_launch(b):
     workgroups wait on each other, so they must all be resident at once; the default plain launch
     sizes its grid to the device's resident capacity, which holds when nothing else occupies the
     compute units. A cooperative launch guarantees it for callers that share the GPU with other
-    streams or processes, at ~14-19 us per call (same results bit for bit). No counterpart in the
-    reference."""
+    streams or processes, at ~14-19 us per call (same results bit for bit); launches whose
+    workgroups wait for nothing (L1 alone, L2 before a combine launch) stay plain. No counterpart in
+    the reference."""
     c = getattr(b, "cooperative", None)
     return bool(c) if c is not None else os.environ.get("DG_MEGA_COOPERATIVE", "0") == "1"
 

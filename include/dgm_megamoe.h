@@ -320,7 +320,9 @@ typedef struct DgmMoeArgs {
    * to what the device keeps resident, which holds when no other work occupies the compute
    * units. DGM_LAUNCH_COOPERATIVE launches it cooperatively (hipLaunchCooperativeKernel), which
    * guarantees co-residency for callers that share the GPU with other streams or processes, at
-   * a cost of ~14-19 us per call on MI355X. No counterpart in the reference (a plain launch). */
+   * a cost of ~14-19 us per call on MI355X. Launches whose workgroups wait for nothing (L1 alone, and
+   * L2 before a combine launch: the MXFP4 / MXFP8 / FP8F128 split and beyond-limit calls) stay
+   * plain. No counterpart in the reference (a plain launch). */
   int32_t launch_flags;
 } DgmMoeArgs;
 
