@@ -755,7 +755,8 @@ DGM_DEV void slab_store(S& s, const SlabRegs<KT, ACT, COHERENT, MIDL>& r) {
 // [4] L2 units done, [5] exit; [6] wall ticks in L1 K loops (matrix-core ops, including the
 // waits for their weight tiles), [7] wall ticks in L1 epilogues. With the in-kernel frontend,
 // [6] and [7] are instead wall clock at: this workgroup's router and cast work done (its
-// stores issued), and the grid-wide arrival passed.
+// stores issued), and the grid-wide arrival passed. Where L1 and L2 are launches of their own, each has
+// rows of its own, L2's behind L1's (launch_fused_t).
 DGM_DEV long long wall_clock() { return (long long)__builtin_amdgcn_s_memrealtime(); }
 
 // FEIN: the router, token flags and activation cast run in this launch (p.fe_in); the rows they
@@ -2153,7 +2154,7 @@ GridCache& grid_cache() {
 }
 
 template <int KT1, int KT2, int ACT, int FORM>
-int launch_fused_t(const FusedParams& prm, int slot, hipStream_t stream, bool coop) {
+int launch_fused_t(FusedParams prm, int slot, hipStream_t stream, bool coop) {
   GridCache& gc = grid_cache();
   int& nb = gc.blocks[slot][ACT][FORM];
   if (nb == 0) {
@@ -2165,12 +2166,16 @@ int launch_fused_t(const FusedParams& prm, int slot, hipStream_t stream, bool co
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     nb = per_cu * (cus > 0 ? cus : 256);
   }
+  // (an L2 launch's stamp rows follow those of the L1 launch before it, which had as many workgroups)
+  if (prm.stamp_rows > 0 && !(prm.phases & 1)) {
+    prm.stamp_rows = prm.stamp_rows > nb ? prm.stamp_rows - nb : 0;
+    prm.stamps += (size_t)nb * 8;
+  }
   gc.last[slot][ACT] = nb;
   gc.form[slot][ACT] = FORM;
   if (coop) {
     // (the grid is the device's resident capacity, which a cooperative launch requires)
-    FusedParams arg = prm;
-    void* args[] = {&arg};
+    void* args[] = {&prm};
     const hipError_t e = hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&k_megamoe<KT1, KT2, ACT, FORM>),
                                                     dim3(nb), dim3(FT), args, 0, stream);
     if (e != hipSuccess) {

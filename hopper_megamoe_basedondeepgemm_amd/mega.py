@@ -748,7 +748,9 @@ def qoq_mega_moe_split(y, l1_weights, l2_weights, sym_buffer, *args, **kwargs):
 
 
 def fused_workgroups(b):
-    """Workgroups of the persistent kernel for this buffer's shape (after its first launch)."""
+    """Workgroups of the persistent kernel for this buffer's shape (after its first launch): the
+    ``phase_stamps`` rows of a one-launch call. A call of several launches (split, or beyond the
+    one-launch limits) stamps as many rows for L1 and, behind them, as many for L2."""
     return _lib.load().dgm_fused_workgroups(b.hidden, b.intermediate_hidden, b.act_code)
 
 

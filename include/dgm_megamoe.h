@@ -275,7 +275,11 @@ typedef struct DgmMoeArgs {
   const DgmBufferLayout* layout;
   int64_t* phase_stamps;  /* optional [phase_stamp_rows, 8] wall-clock stamps (phase_stamps of
                              deep_gemm/mega/fused.py:97); NULL = off. Workgroups beyond
-                             phase_stamp_rows record nothing. */
+                             phase_stamp_rows record nothing. 100 MHz wall clock: [0] entry, [1] dispatch
+                             table ready, [2] L1 units done, [3] first L1 arrival waited for, [4] L2 units
+                             done, [5] exit; [6], [7] ticks in L1 K loops and epilogues. A call of
+                             several launches: rows [0, G) are the L1 launch's, [G, 2 G) the L2 launch's
+                             (G = dgm_fused_workgroups) */
   int32_t phase_stamp_rows;
   const float* w1_row_scales; /* QoQ: s1 [E_local, 2I] (dgm_transform_qoq_weights order); else unused */
   const float* w2_row_scales; /* QoQ: s1 [E_local, H]; else unused */

@@ -45,3 +45,45 @@ def test_cooperative_option_same_results(fmt, M, split):
         out.append(_call(dgm, l1, l2, buf, M, split))
     for u, v in zip(*out):
         assert torch.equal(u, v)
+
+
+@pytest.mark.parametrize("fmt,M,split", [("mxfp8", 20, True), ("mxfp8", 300, False), ("qoq", 20, True)])
+def test_phase_stamps_of_both_launches(fmt, M, split):
+    """The L1 launch stamps the first rows and the L2 launch as many behind them, each in phase order
+    within the launch, L2's launch entered once every workgroup of L1's was done; y does not
+    change, and a stamp array that ends inside either launch's rows is not written past."""
+    need_gpu()
+    import hopper_megamoe_basedondeepgemm_amd as dgm
+    print(f"stamps of both launches fmt={fmt} M={M} split={split}", flush=True)
+    if fmt == "qoq":
+        from tests.test_gpu_qoq import make_qoq_weights
+        _, _, buf = _filled(dgm, "mxfp8", M)
+        idx, w = buf.topk_idx.clone(), buf.topk_weights.clone()
+        (l1, l2), kw = make_qoq_weights(E, H, I, 22)[0], {"fmt": "qoq"}
+        buf = dgm.get_fused_symm_buffer_for_mega_moe(None, E, M, TOPK, H, I, act_format=fmt)
+        x = torch.randn((M, H), generator=torch.Generator(device="cuda").manual_seed(M), device="cuda").bfloat16()
+        dgm.mega._cast_into(buf, x, fmt)
+        buf.topk_idx.copy_(idx)
+        buf.topk_weights.copy_(w)
+    else:
+        l1, l2, buf = _filled(dgm, fmt, M)
+        kw = {}
+    y0, s0 = _call(dgm, l1, l2, buf, M, split, **kw)
+    st = torch.zeros((2048, 8), dtype=torch.int64, device="cuda")
+    y1, s1 = _call(dgm, l1, l2, buf, M, split, phase_stamps=st, **kw)
+    assert torch.equal(y0, y1) and torch.equal(s0, s1)
+    G = dgm.mega.fused_workgroups(buf)
+    a = st.cpu().numpy()
+    assert 0 < 2 * G < 2048 and (a[2 * G:] == 0).all()
+    one, two = a[:G], a[G:2 * G]
+    for r in (one, two):
+        assert (r[:, 0] > 0).all() and (r[:, 1] >= r[:, 0]).all() and (r[:, 2] >= r[:, 1]).all()
+        assert (r[:, 4] >= r[:, 2]).all() and (r[:, 5] >= r[:, 4]).all()
+        assert (r[:, 6] + r[:, 7] <= r[:, 5] - r[:, 0]).all()
+    assert two[:, 0].min() >= one[:, 2].max()
+    assert (one[:, 6] > 0).any() and (two[:, 6:] == 0).all()          # (L1 K loops run in the first alone)
+    for n in (G + G // 2, G // 2):
+        part = torch.zeros((2 * G, 8), dtype=torch.int64, device="cuda")
+        y2, _ = _call(dgm, l1, l2, buf, M, split, phase_stamps=part[:n], **kw)
+        p = part.cpu().numpy()
+        assert torch.equal(y0, y2) and (p[:n, 0] > 0).all() and (p[n:] == 0).all()
