@@ -588,8 +588,9 @@ int dgm_fused_launch_ws(const DgmMoeArgs* A, int phases, const DgmWorkspace& w, 
   uint8_t* buf = (uint8_t*)A->buffer;
   {
     const int fast = (A->fe_flags & DGM_FE_FORCE_BALANCED) ? SELECT_IN_MEGA_FAST_BALANCED : SELECT_IN_MEGA_FAST_TOKENS;
-    // (the large-batch form reads the top-k)
-    const bool sel = (A->fe_in_mega || (A->select_in_mega && A->num_tokens <= fast)) && (phases & 1) && fused_fits(A);
+    // (the large-batch form reads the top-k; the kernel's selection has no raw weights)
+    const bool raw = (A->fe_flags & DGM_FE_RAW_WEIGHTS) && !(A->fe_flags & DGM_FE_FORCE_BALANCED);
+    const bool sel = (A->fe_in_mega || (A->select_in_mega && A->num_tokens <= fast && !raw)) && (phases & 1) && fused_fits(A);
     if (A->select_in_mega && !sel && (phases & 1)) {
       int st = materialize_topk(A, buf, L, stream);
       if (st) return st;

@@ -87,3 +87,30 @@ def test_phase_stamps_of_both_launches(fmt, M, split):
         y2, _ = _call(dgm, l1, l2, buf, M, split, phase_stamps=part[:n], **kw)
         p = part.cpu().numpy()
         assert torch.equal(y0, y2) and (p[:n, 0] > 0).all() and (p[n:] == 0).all()
+
+
+@pytest.mark.parametrize("flags", ["raw", "raw and forced-balanced"])
+@pytest.mark.parametrize("M", [5, 12])          # within and beyond the in-kernel selection's tokens
+@pytest.mark.parametrize("fmt,split", [("mxfp4", True), ("mxfp8", True), ("fp8f128", True), ("mxfp8", False)])
+def test_raw_weights_selected_by_the_layer_call(fmt, split, M, flags):
+    """DGM_FE_RAW_WEIGHTS with the top-k left to the layer call: the routing and y of the same top-k
+    selected beforehand."""
+    need_gpu()
+    import ctypes
+    import hopper_megamoe_basedondeepgemm_amd as dgm
+    from hopper_megamoe_basedondeepgemm_amd import _lib
+    print(f"raw weights fmt={fmt} split={split} M={M} {flags}", flush=True)
+    bits = _lib.FE_RAW_WEIGHTS | (_lib.FE_FORCE_BALANCED if "forced" in flags else 0)
+    l1, l2, buf = _filled(dgm, fmt, M)
+    logits = torch.randn((M, E), generator=torch.Generator(device="cuda").manual_seed(31), device="cuda").bfloat16()
+    out = []
+    for left in (0, _lib.FE_SELECT_IN_MEGA):
+        _lib.check(_lib.load().dgm_router_logits_topk_launch(
+            _lib.ptr(logits), M, E, TOPK, bits | left, 0, _lib.ptr(buf.buffer), ctypes.byref(buf.layout), _lib.stream()))
+        buf._fe_select = (bits, 0) if left else None
+        y, stats = _call(dgm, l1, l2, buf, M, split)
+        out.append((y, stats, buf.topk_idx.clone(), buf.topk_weights.clone()))
+    for u, v in zip(*out):
+        assert torch.equal(u, v)
+    if "forced" not in flags:
+        assert torch.equal(out[1][3], logits.float().sort(dim=1, descending=True).values[:, :TOPK])
