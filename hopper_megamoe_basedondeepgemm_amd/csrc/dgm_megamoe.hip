@@ -36,11 +36,17 @@ namespace {
 // its barrier cost 1.1-1.7 us more than the hidden-row reads they save).
 constexpr int FE_ROUTER_TILE = 8;         // tokens per router workgroup in the tiled form
 constexpr int FE_TILE_MIN_TOKENS = 64;
-// Matrix-core router tiles (router_tile_mm) from 112 tokens (seven 16-token tiles) on: 128 tokens
-// 12.6 us against 20.0, 100 tokens 12.8 against 17.9, 64 tokens 12.4 against 13.0, 48 tokens 12.4
-// against 12.8, 32 tokens 12.4 against 10.0 (with the selection launch). Between 48 and 111 tokens
-// the eight-token rows stay: fable_frontend_router_ctas publishes their workgroup counts.
-constexpr int FE_MM_MIN_TOKENS = 112;
+// Matrix-core router tiles (router_tile_mm) beyond 64 tokens, for hidden sizes beyond 1024 only with more
+// than 64 tiles of 16 tokens x 16 experts: a tile alone takes as long as a whole round of them (its
+// K loop), which fewer tiles do not shorten, while the rows of eight tokens get shorter. Frontend +
+// selection launch, us, rows against tiles:
+//   H 3072, E 384: 80 tokens 16.8 / 12.7, 100 17.9 / 12.9, 128 20.3 / 12.8, 512 61.7 / 26.6
+//           E 128: 128 tokens (64 tiles) 11.4 / 12.4, 160 (80) 12.9 / 12.8, 256 16.7 / 13.0
+//           E 48: 128 tokens (24 tiles) 10.6 / 12.3, 384 (72) 13.0 / 12.9, 512 15.1 / 13.2
+//   H 4096, E 128: 112 tokens (56 tiles) 12.7 / 14.7, 160 (80) 17.7 / 14.7; H 2048: 10.1 / 10.5, 11.0 / 10.6
+//   H 1024, E 8: 80 tokens 8.3 / 7.5, E 48: 8.7 / 8.3; H 512, E 8: 8.1 / 6.4, E 384: 8.9 / 7.4
+// Up to 64 tokens the rows stay (E 384 H 3072, 64 tokens 13.1 / 12.7, 32 tokens 10.2 / 12.3).
+constexpr int FE_MM_MIN_TOKENS = 65, FE_MM_MIN_TILES = 65, FE_MM_ANY_TILES_HIDDEN = 1024;
 // Phase stamps (the reference's DG_FE_STAMPS, deep_gemm/mega/__init__.py:743-756): with stamps
 // non-null, workgroup b = blockIdx.y * gridDim.x + blockIdx.x < stamp_rows writes row b of 8
 // int64: [0] entry, [3] (router rows) keys and logits stored by all four waves, [5] (cast rows)
@@ -110,7 +116,7 @@ __global__ void __launch_bounds__(256) k_frontend(const uint16_t* __restrict__ x
   }
 }
 
-// The frontend from FE_MM_MIN_TOKENS tokens on: workgroups [0, nr) are router tiles of 16 tokens x
+// The frontend by router tiles (fe_mm): workgroups [0, nr) are router tiles of 16 tokens x
 // 16 experts on the matrix cores (router_tile_mm, experts fastest: with E % 128 == 0 an XCD then
 // keeps one share of the router weights in its L2), the rest cast.
 template <int J>
@@ -369,10 +375,15 @@ extern "C" {
 
 }  // extern "C"
 
-static bool fe_mm(int num_tokens, bool router) { return router && num_tokens >= FE_MM_MIN_TOKENS; }
+static int fe_tiles(int num_tokens, int num_experts) { return ((num_experts + 15) / 16) * ((num_tokens + 15) / 16); }
+// Whether the router runs as matrix-core tiles
+static bool fe_mm(int num_tokens, int hidden, int num_experts, bool router) {
+  return router && num_tokens >= FE_MM_MIN_TOKENS &&
+         (hidden <= FE_MM_ANY_TILES_HIDDEN || fe_tiles(num_tokens, num_experts) >= FE_MM_MIN_TILES);
+}
 
-// The frontend launch's grid: router rows (4 experts x 4 tokens per workgroup, 8 tokens from
-// FE_TILE_MIN_TOKENS on) and, beside them, cast rows of one cast lane per thread (QoQ: one wave
+// The frontend launch's grid: router tiles (fe_mm) or rows (4 experts x 4 tokens per workgroup, 8
+// tokens from FE_TILE_MIN_TOKENS on) and, beside them, cast rows of one cast lane per thread (QoQ: one wave
 // per token).
 static dim3 fe_grid(int num_tokens, int hidden, int num_experts, int act_format, int flags, bool router) {
   const int rx = (num_experts + 3) / 4;
@@ -381,9 +392,8 @@ static dim3 fe_grid(int num_tokens, int hidden, int num_experts, int act_format,
                                : act_format == DGM_ACT_FP8F128 ? (int64_t)num_tokens * (hidden / 128) * 32
                                                                : (int64_t)num_tokens * (hidden / 32) * 8;
   const int64_t cast_rows = (flags & DGM_FE_NO_CAST) ? 0 : (cast_threads + (int64_t)rx * 256 - 1) / ((int64_t)rx * 256);
-  if (fe_mm(num_tokens, router))
-    return dim3(((num_experts + 15) / 16) * ((num_tokens + 15) / 16) +
-                ((flags & DGM_FE_NO_CAST) ? 0 : (int)((cast_threads + 511) / 512)));
+  if (fe_mm(num_tokens, hidden, num_experts, router))
+    return dim3(fe_tiles(num_tokens, num_experts) + ((flags & DGM_FE_NO_CAST) ? 0 : (int)((cast_threads + 511) / 512)));
   const int rtok = num_tokens >= FE_TILE_MIN_TOKENS ? FE_ROUTER_TILE : 4;
   return dim3(rx, (router ? (num_tokens + rtok - 1) / rtok : 0) + (int)cast_rows);
 }
@@ -427,7 +437,7 @@ int dgm_router_topk_launch_stamped(const void* hidden_bf16, const void* router_w
   uint8_t* buf = (uint8_t*)buffer;
   const int J = hidden / 512;
   const int router = router_weight_bf16 ? 1 : 0;
-  const bool tiled = num_tokens >= FE_TILE_MIN_TOKENS, mm = fe_mm(num_tokens, router != 0);
+  const bool tiled = num_tokens >= FE_TILE_MIN_TOKENS, mm = fe_mm(num_tokens, hidden, num_experts, router != 0);
   const dim3 rg = fe_grid(num_tokens, hidden, num_experts, act_format, flags, router != 0);
   long long* stamp_ptr = (long long*)stamps;
   const uint16_t* x = (const uint16_t*)hidden_bf16;
@@ -439,7 +449,7 @@ int dgm_router_topk_launch_stamped(const void* hidden_bf16, const void* router_w
   if (mm)                                                                                                    \
     hipLaunchKernelGGL((k_frontend_mm<JJ>), rg, dim3(512), 0, stream, x, w, num_tokens, num_experts, act_format, \
                        logits, keys, zero_unrouted, buf + L->x, buf + L->x_sf,                               \
-                       ((num_experts + 15) / 16) * ((num_tokens + 15) / 16), stamp_ptr, stamp_rows);         \
+                       fe_tiles(num_tokens, num_experts), stamp_ptr, stamp_rows);                            \
   else if (tiled)                                                                                            \
     hipLaunchKernelGGL((k_frontend<JJ, FE_ROUTER_TILE>), rg, dim3(256), 0, stream, x, w, num_tokens, num_experts, \
                        act_format, logits, keys, zero_unrouted, buf + L->x, buf + L->x_sf, router, stamp_ptr, \

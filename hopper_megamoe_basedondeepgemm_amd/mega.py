@@ -287,7 +287,9 @@ def transform_weights_for_mega_moe(l1, l2):
 # ----------------------------------------------------------------------------- frontend
 SELECT_IN_MEGA_MAX_TOKENS = 64    # every workgroup of the fused kernel reads all tokens' logits
 FE_ROUTER_TILE_MIN_TOKENS = 64    # the frontend's router rows of 8 tokens (csrc FE_TILE_MIN_TOKENS)
-FE_ROUTER_MM_MIN_TOKENS = 112     # its 16 x 16 router tiles on the matrix cores (csrc FE_MM_MIN_TOKENS)
+# its 16 x 16 router tiles on the matrix cores: from these tokens and tiles on; any tiles up to this
+# hidden size (csrc FE_MM_MIN_TOKENS, FE_MM_MIN_TILES, FE_MM_ANY_TILES_HIDDEN)
+FE_ROUTER_MM_MIN_TOKENS, FE_ROUTER_MM_MIN_TILES, FE_ROUTER_MM_ANY_TILES_HIDDEN = 65, 65, 1024
 # csrc/fable_frontend.h kFEPath* (deep_gemm/mega/__init__.py:593): the launch-shape families of the
 # reference's frontend. Here one router kernel serves every shape; fable_frontend_path names the
 # family whose options apply (FE_PATH_CC: select_in_mega and zero-row unrouting available).
@@ -306,9 +308,11 @@ def fable_frontend_router_ctas(m: int, e: int, h: int = 3072, topk: int = 8) -> 
     """deep_gemm/mega/__init__.py:653: router workgroups of the frontend launch for (m, h, e,
     topk): four experts per workgroup (one wave each) over 4 tokens, or over 8 tokens from
     FE_ROUTER_TILE_MIN_TOKENS on (the 8 hidden rows staged in LDS and shared by the waves); 16
-    experts over 16 tokens from FE_ROUTER_MM_MIN_TOKENS on (matrix cores)."""
-    if m >= FE_ROUTER_MM_MIN_TOKENS:
-        return ((e + 15) // 16) * ((m + 15) // 16)
+    experts over 16 tokens (matrix cores) from FE_ROUTER_MM_MIN_TOKENS on, where these tiles are at
+    least FE_ROUTER_MM_MIN_TILES or h is at most FE_ROUTER_MM_ANY_TILES_HIDDEN."""
+    tiles = ((e + 15) // 16) * ((m + 15) // 16)
+    if m >= FE_ROUTER_MM_MIN_TOKENS and (tiles >= FE_ROUTER_MM_MIN_TILES or h <= FE_ROUTER_MM_ANY_TILES_HIDDEN):
+        return tiles
     return ((e + 3) // 4) * ((m + 7) // 8 if m >= FE_ROUTER_TILE_MIN_TOKENS else (m + 3) // 4)
 
 

@@ -22,3 +22,18 @@ def test_launches_that_wait_on_other_workgroups(tmp_path):
     (phases 1) nor L2 before a combine launch (2 | 4). A cooperative launch is made for these only."""
     cases = {(1, 0): 0, (6, 0): 0, (2, 0): 1, (3, 0): 1, (1, 1): 1, (3, 1): 1}
     assert _eval(tmp_path, [f"fused_launch_waits({p}, {f})" for p, f in cases]) == list(cases.values())
+
+
+def test_router_tiles_where_they_are_enough():
+    """The frontend's router workgroups: rows up to 64 tokens and where tiles would be few, tiles
+    beyond; the published count is the launch's."""
+    from hopper_megamoe_basedondeepgemm_amd import _lib, mega
+    launch = lambda m, e, h: _lib.load().dgm_frontend_workgroups(m, h, e, 1, _lib.FE_NO_CAST, 1)
+    rows = lambda m, e: ((e + 3) // 4) * ((m + 7) // 8 if m >= 64 else (m + 3) // 4)
+    tiles = lambda m, e: ((e + 15) // 16) * ((m + 15) // 16)
+    for h in (512, 1024, 2048, 3072, 4096):
+        for e in (8, 16, 20, 48, 128, 384, 1000):
+            for m in (1, 63, 64, 65, 80, 81, 111, 112, 128, 129, 256, 512):
+                few = m <= 64 or (h > 1024 and tiles(m, e) <= 64)
+                assert launch(m, e, h) == mega.fable_frontend_router_ctas(m, e, h) == (rows if few else tiles)(m, e), (m, e, h)
+    assert launch(128, 48, 3072) == 192 and launch(128, 384, 3072) == 192
