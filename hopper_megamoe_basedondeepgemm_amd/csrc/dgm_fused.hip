@@ -2210,15 +2210,13 @@ bool use_tail(const FusedParams& prm) {
   return !prm.fe_in && (prm.phases & 1) && (long long)prm.M * prm.topk <= 32 && (prm.debug & 16);
 }
 
-// The large-batch form where the plain form's tables end (1024 routes, 256 tokens, 512 local experts).
-bool use_big(const FusedParams& prm) {
-  return (long long)prm.M * prm.topk > FUSED_MAX_ROUTES || prm.M > FUSED_MAX_TOKENS || prm.E_local > FUSED_MAX_LOCAL;
-}
-
 template <int KT1, int KT2, int ACT>
 int launch_fused_fe(const FusedParams& prm, int slot, hipStream_t stream, bool coop) {
-  if constexpr (ACT == DGM_ACT_MXFP4 || ACT == DGM_ACT_MXFP8 || ACT == DGM_ACT_FP8F128) {
-    if (use_big(prm)) return launch_fused_t<KT1, KT2, ACT, FORM_BIG>(prm, slot, stream, coop);
+  if (fused_needs_big(prm.M, prm.topk, prm.E_local)) {
+    constexpr bool wide = ACT == DGM_ACT_MXFP4 || ACT == DGM_ACT_MXFP8 || ACT == DGM_ACT_FP8F128;
+    DGM_CHECK_ARG(fused_big_runs(prm.M, prm.topk, prm.E_local, wide, prm.phases, prm.select != 0, prm.fe_in != 0),
+                  "large-batch form: MXFP4 / MXFP8 / FP8F128, one phase per launch");
+    if constexpr (wide) return launch_fused_t<KT1, KT2, ACT, FORM_BIG>(prm, slot, stream, coop);
   }
   if constexpr (ACT == DGM_ACT_MXFP4 || ACT == DGM_ACT_MXFP8) {
     if (use_early(prm, ACT)) return launch_fused_t<KT1, KT2, ACT, FORM_EARLY>(prm, slot, stream, coop);

@@ -87,6 +87,17 @@ struct FusedParams {
                             // bit 4: tail half units
 };
 
+// The large-batch form (FORM_BIG): calls whose tables the other forms do not hold, and the launches of it
+// that can run: one phase each (L1, or L2 before a combine launch: its L2 units wait for no L1 unit),
+// the top-k selected beforehand, in a format that has the form.
+constexpr bool fused_needs_big(int M, int topk, int E_local) {
+  return (long long)M * topk > FUSED_MAX_ROUTES || M > FUSED_MAX_TOKENS || E_local > FUSED_MAX_LOCAL;
+}
+constexpr bool fused_big_runs(int M, int topk, int E_local, bool wide_format, int phases, bool select, bool fe_in) {
+  return wide_format && (phases == 1 || phases == 6) && !select && !fe_in &&
+         (long long)M * topk <= FUSED_BIG_ROUTES && E_local <= FUSED_BIG_LOCAL;
+}
+
 // Whether workgroups of a launch wait on each other (the in-kernel frontend's grid-wide arrival, L2's
 // wait for L1 units, the combine's for L2 units) and so must all be resident at once: not L1 alone,
 // and not L2 without the combine.

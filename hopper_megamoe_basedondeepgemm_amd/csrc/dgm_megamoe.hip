@@ -575,8 +575,7 @@ int dgm_check_fused_args(const DgmMoeArgs* A) {
 // activations run the large-batch form, one launch per phase, whose tables hold every call that a
 // buffer layout admits.
 static bool fused_fits(const DgmMoeArgs* A) {
-  return A->num_tokens * A->topk <= FUSED_MAX_ROUTES && A->num_local_experts <= FUSED_MAX_LOCAL &&
-         A->num_tokens <= FUSED_MAX_TOKENS && A->hidden / 64 <= FUSED_MAX_NB64;
+  return !fused_needs_big(A->num_tokens, A->topk, A->num_local_experts) && A->hidden / 64 <= FUSED_MAX_NB64;
 }
 // One launch of the persistent kernel running `phases` (FusedParams::phases) of the layer, with
 // the buffer's own workspace views.

@@ -37,3 +37,17 @@ def test_router_tiles_where_they_are_enough():
                 few = m <= 64 or (h > 1024 and tiles(m, e) <= 64)
                 assert launch(m, e, h) == mega.fable_frontend_router_ctas(m, e, h) == (rows if few else tiles)(m, e), (m, e, h)
     assert launch(128, 48, 3072) == 192 and launch(128, 384, 3072) == 192
+
+
+def test_large_batch_form_runs_one_phase_of_its_formats(tmp_path):
+    """Beyond the plain form's tables only launches whose L2 units need no L1 unit of the same launch,
+    of the formats that have the form, within its own tables."""
+    needs = {(256, 4, 512): 0, (129, 8, 1): 1, (257, 1, 1): 1, (1, 1, 513): 1}
+    runs = {(512, 8, 1024, 1, 1, 0, 0): 1, (512, 8, 1024, 1, 6, 0, 0): 1,
+            (512, 8, 1024, 1, 3, 0, 0): 0, (512, 8, 1024, 1, 2, 0, 0): 0,      # L2 with its combine
+            (512, 8, 1024, 0, 1, 0, 0): 0,                                     # QoQ, NVFP4
+            (512, 8, 1024, 1, 1, 1, 0): 0, (512, 8, 1024, 1, 1, 0, 1): 0,      # top-k or frontend in the kernel
+            (513, 8, 1024, 1, 1, 0, 0): 0, (512, 8, 1025, 1, 1, 0, 0): 0}      # beyond its tables
+    fmt = lambda name, a: f"{name}({', '.join(map(str, a))})"
+    assert _eval(tmp_path, [fmt("fused_needs_big", a) for a in needs] + [fmt("fused_big_runs", a) for a in runs]) == \
+        list(needs.values()) + list(runs.values())
