@@ -175,9 +175,15 @@ def check(status):
         raise RuntimeError(f"dgm error {status}: {msg}")
 
 
+# The current stream's handle itself (a torch.cuda.Stream object for it costs 3 us per call). A private
+# name of torch: None where this torch has none.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream():
-    # (the current stream's handle itself: a torch.cuda.Stream object for it costs 3 us per call)
-    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
+    if _raw_stream is None:
+        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return ctypes.c_void_p(_raw_stream(torch.cuda.current_device()))
 
 
 def ptr(t):

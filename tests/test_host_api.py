@@ -110,3 +110,15 @@ def test_route_to_token_multiply_is_exact_within_the_host_limits():
         m = (0x100000 + d - 1) // d
         assert np.array_equal((r * np.uint64(m)) >> np.uint64(20), r // np.uint64(d)), d
         assert int(r[-1]) * m < 2 ** 32          # (the kernel multiplies in 32 bits)
+
+
+def test_stream_handle_with_and_without_the_private_name(monkeypatch):
+    """The current stream's handle, from torch's private function or, without it, its public one."""
+    class Stream:
+        cuda_stream = 0x5678
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 3)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: Stream)
+    monkeypatch.setattr(_lib, "_raw_stream", lambda dev: 0x1230 + dev)
+    assert _lib.stream().value == 0x1233
+    monkeypatch.setattr(_lib, "_raw_stream", None)
+    assert _lib.stream().value == 0x5678
