@@ -146,3 +146,19 @@ def oracle_routes_parallel(x_dq, idx, w, experts, deq1, deq2, expert_begin, E_lo
 def active_local_experts(idx, expert_begin, E_local):
     loc = np.asarray(idx) - expert_begin
     return sorted({int(v) for v in loc.ravel() if 0 <= v < E_local and v + expert_begin >= 0})
+
+
+def launch_count(fn):
+    """The kernels (and copies, if any) that fn enqueues on the current stream: the nodes of a HIP graph
+    that captures them (not replayed). Call fn once before, so that nothing is set up inside."""
+    import ctypes
+    import re
+    path = next(m.group(1) for m in (re.search(r"(/\S*libamdhip64\S*)", l) for l in open("/proc/self/maps")) if m)
+    hip = ctypes.CDLL(path)                   # (the runtime that this process has loaded)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        fn()
+    n = ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+    return n.value

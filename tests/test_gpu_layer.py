@@ -168,7 +168,8 @@ def test_second_ep_rank_and_replay():
 
 @pytest.mark.parametrize("fmt", ["mxfp4", "mxfp8"])
 def test_split_matches_fused(fmt):
-    """The split API (separate launches) gives the fused kernel's result bit for bit."""
+    """The split API (the same kernel, L1 and L2 as launches of their own) gives the one launch's result
+    bit for bit."""
     need_gpu()
     import hopper_megamoe_basedondeepgemm_amd as dgm
     weights = make_weights(48, 3072, 1280, 601)
@@ -272,7 +273,7 @@ def test_persistent_kernel_at_its_limits(fmt):
 
 def test_large_batch_beyond_fused_limits():
     """200 tokens at top-8: 1600 routes exceed the persistent kernel's 1024, so the fused entry
-    point runs the split path (dispatch, L1, L2, combine kernels); frontend, pool and y as
+    point runs the split call's launches (dispatch + L1, L2, combine); frontend, pool and y as
     everywhere else."""
     need_gpu()
     r = run_layer(200, 16, 16, 0, 512, 256, 8, "mxfp4", seed=950, zero_rows=(7,))
