@@ -43,7 +43,7 @@ static constexpr inline size_t dgm_pool_bytes(int E_local, int max_routes) {
 
 // Device memory the persistent kernel uses beyond its inputs and outputs: the dispatch table,
 // the L1 -> L2 rows and scales, the bf16 route outputs ([topk][part_rows][H]) and the int32
-// counters (which start at zero and are returned to zero by every launch).
+// counters (zero before the first launch; every launch clears the set that the next one uses).
 struct DgmWorkspace {
   uint8_t* pool;
   uint8_t* mid;
@@ -77,6 +77,7 @@ int dgm_check_layout_call(const DgmBufferLayout* L, int num_tokens, int topk, in
 // Host-side checks of a fused-layer call (0, or DGM_ERR_INVALID_ARGUMENT with the message set).
 int dgm_check_fused_args(const DgmMoeArgs* A);
 // One launch of the persistent kernel over the workspace w, running `phases` of the layer
-// (1: dispatch + L1, 2: L2 + combine, 3: both); the top-k selection launch first when the
+// (1: dispatch + L1, 2: L2 + combine, 3: both, 2 | 4: L2 without the combine; beyond the plain form's
+// limits 1 and 2 | 4 only); the top-k selection launch first when the
 // call selects from keys above the in-kernel selection's token count.
 int dgm_fused_launch_ws(const DgmMoeArgs* A, int phases, const DgmWorkspace& w, hipStream_t stream);

@@ -50,16 +50,6 @@ DGM_DEV uint32_t e2m1_ties_down(float x) {
   uint32_t c = e2m1_mag_code(fabsf(x));
   return c | ((x < 0.f && c != 0u) ? 8u : 0u);
 }
-// Packer rule: magnitude clamped to 6, sign bit for every negative input (-0 code possible).
-DGM_DEV uint32_t e2m1_bucketize(float x) {
-  uint32_t c = e2m1_mag_code(fminf(fabsf(x), 6.0f));
-  return c | (x < 0.f ? 8u : 0u);
-}
-DGM_DEV float e2m1_value(uint32_t nib) {
-  const float mag[8] = {0.f, 0.5f, 1.f, 1.5f, 2.f, 3.f, 4.f, 6.f};
-  float v = mag[nib & 7u];
-  return (nib & 8u) ? -v : v;
-}
 
 // ---------------------------------------------------------------- E8M0
 // Smallest power of two >= |x| by exponent bits, exponent clamped to [1, 254].
@@ -69,12 +59,8 @@ DGM_DEV uint32_t ceil_ue8m0_code(float x) {
   return e < 1u ? 1u : (e > 254u ? 254u : e);
 }
 DGM_DEV float e8m0_value(uint32_t code) { return __uint_as_float(code << 23); }   // code >= 1
-// 2^(code-127) including code 0 (2^-127, subnormal).
-DGM_DEV float e8m0_value_any(uint32_t code) {
-  return code == 0u ? __uint_as_float(0x00400000u) : __uint_as_float(code << 23);
-}
 // 2^(127 - code): the exact reciprocal of the E8M0 value (code 254 gives the subnormal 2^-127),
-// so x * e8m0_inv(code) == x / e8m0_value_any(code) bit for bit.
+// so x * e8m0_inv(code) is x divided by the code's value (code 0: 2^-127) bit for bit.
 DGM_DEV float e8m0_inv(uint32_t code) {
   return code >= 254u ? __uint_as_float(0x00400000u) : __uint_as_float((254u - code) << 23);
 }
@@ -245,14 +231,6 @@ DGM_DEV void select_topk_wave(LoadKey load, int E, int topk, bool balanced, int 
   else if (nk <= 6) select_topk_wave_nk<6>(load, E, topk, lane, idx, wt);
   else if (nk <= 8) select_topk_wave_nk<8>(load, E, topk, lane, idx, wt);
   else select_topk_wave_nk<16>(load, E, topk, lane, idx, wt);
-}
-
-// ---------------------------------------------------------------- scopes / atomics
-DGM_DEV int atomic_add_acqrel_agent(int* p, int v) {
-  return __hip_atomic_fetch_add(p, v, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-}
-DGM_DEV int atomic_load_acquire_agent(const int* p) {
-  return __hip_atomic_load(p, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ---------------------------------------------------------------- matrix cores

@@ -30,8 +30,8 @@
 // launch runs L1 and one L2 without the combine, which is then a kernel of its own: no workgroup of
 // those waits on another.
 //
-// Hand-offs between workgroups go through HBM with agent-coherent accesses only: the data
-// (intermediate codes and scales, bf16 route outputs) is written with relaxed agent-scope
+// Hand-offs between workgroups of one launch go through HBM with agent-coherent accesses only (the
+// large-batch form hands over to its next launch, with ordinary ones): the data (intermediate codes and scales, bf16 route outputs) is written with relaxed agent-scope
 // atomic stores (write-through, "sc1") and read with agent-scope atomic loads, and the
 // producer's stores have completed (s_waitcnt) before it bumps an arrival counter. No
 // agent-scope release/acquire fence is used: on this GPU those write back / invalidate a
@@ -86,15 +86,6 @@ DGM_DEV void st_handoff8(uint8_t* p, uint8_t v) {
 }
 DGM_DEV uint64_t ld_agent64(const void* p) {
   return __hip_atomic_load((const uint64_t*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-DGM_DEV uint32_t ld_agent8(const uint8_t* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// Compiler-only ordering point: memory operations after it stay after the matrix-core ops
-// that produced `acc` (otherwise the next unit's tile loads may be hoisted above them and
-// need a second register set).
-DGM_DEV void after_mfma(v4f acc) {
-  asm volatile("" ::"v"(acc[0]), "v"(acc[1]), "v"(acc[2]), "v"(acc[3]) : "memory");
 }
 // all of this wave's memory operations have completed (stores acknowledged)
 DGM_DEV void wait_mem() {
@@ -1439,7 +1430,7 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
           }
         });
       } else if constexpr (F128) {
-        // one chain, as the split path's L1 kernel: per K-tile the block-scaled op with a unit
+        // one chain in K order: per K-tile the block-scaled op with a unit
         // activation scale into a zero accumulator, then acc += s * part with the token's fp32
         // scale s of that K-tile, one tile later (off the op's latency). A compiler ordering
         // point keeps each op after the promote two tiles back (independent ops would otherwise
@@ -1475,9 +1466,8 @@ __global__ void __launch_bounds__(FT) k_megamoe(FusedParams p) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[i] = fmaf(xf_p, prev[i], acc[i]);
       } else {
-        // two chains, K-tiles 0 .. KT1 / 2 - 1 and KT1 / 2 .., summed after the loop: the split
-        // path's L1 kernel sums the same two, so the two paths agree bit for bit for any data.
-        // (TAIL, a half item: each wave runs one of the chains, K half w >> 2, and a K half 0
+        // two chains, K-tiles 0 .. KT1 / 2 - 1 and KT1 / 2 .., summed after the loop, the same in
+        // every form, so that they agree bit for bit for any data. (TAIL, a half item: each wave runs one of the chains, K half w >> 2, and a K half 0
         // wave refills its slots with the next item's tiles: a half item fills the ring once.)
         v4f acc2 = {0.f, 0.f, 0.f, 0.f};
         uint32_t bs = bs0;

@@ -371,10 +371,6 @@ int dgm_check_layout_call(const DgmBufferLayout* L, int num_tokens, int topk, in
   return 0;
 }
 
-extern "C" {
-
-}  // extern "C"
-
 static int fe_tiles(int num_tokens, int num_experts) { return ((num_experts + 15) / 16) * ((num_tokens + 15) / 16); }
 // Whether the router runs as matrix-core tiles
 static bool fe_mm(int num_tokens, int hidden, int num_experts, bool router) {

@@ -93,8 +93,8 @@ DGM_DEV uint32_t lowfirst8(const uint32_t* n) {
 }
 
 // ------------------------------------------------------------------ E2M1 weight codes
-// The packer code (e2m1_bucketize of v / sc clamped to +-6: midpoints go to the smaller magnitude,
-// the sign bit for every negative quotient) of eight elements as one Marlin dword, from the
+// The packer code (of v / sc clamped to +-6: midpoints go to the smaller magnitude, the sign bit for
+// every negative quotient) of eight elements as one Marlin dword, from the
 // conversion instruction, which rounds midpoints to even. inv = 1 / sc, correctly rounded.
 // bf16 / fp16 sources: v / sc is shrunk by 2^-13, so an element on a midpoint b falls below it, and
 // one beyond stays beyond (v has at most 11 significant bits and b sc at most 7, so v > b sc means

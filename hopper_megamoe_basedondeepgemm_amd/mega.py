@@ -291,7 +291,7 @@ FE_ROUTER_TILE_MIN_TOKENS = 64    # the frontend's router rows of 8 tokens (csrc
 # hidden size (csrc FE_MM_MIN_TOKENS, FE_MM_MIN_TILES, FE_MM_ANY_TILES_HIDDEN)
 FE_ROUTER_MM_MIN_TOKENS, FE_ROUTER_MM_MIN_TILES, FE_ROUTER_MM_ANY_TILES_HIDDEN = 65, 65, 1024
 # csrc/fable_frontend.h kFEPath* (deep_gemm/mega/__init__.py:593): the launch-shape families of the
-# reference's frontend. Here one router kernel serves every shape; fable_frontend_path names the
+# reference's frontend. Here the router's kernel follows from the sizes; fable_frontend_path names the
 # family whose options apply (FE_PATH_CC: select_in_mega and zero-row unrouting available).
 FE_PATH_WMMA, FE_PATH_SWAPAB, FE_PATH_CC = 0, 1, 2
 
@@ -764,8 +764,8 @@ FUSED_FORMS = {0: "plain", 1: "in-kernel frontend", 2: "early weight streaming",
 
 def fused_last_form(b):
     """The form the persistent kernel's last launch for this buffer's shape and format ran (a
-    key of ``FUSED_FORMS``; -1 before the first). "large batch" runs beyond 1024 routes or 256 tokens
-    (MXFP4 / MXFP8 / FP8F128 activations). Two opt-in forms, both measured slower than the
+    key of ``FUSED_FORMS``; -1 before the first). "large batch" runs beyond 1024 routes,
+    256 tokens or 512 local experts (MXFP4 / MXFP8 / FP8F128 activations). Two opt-in forms, both measured slower than the
     default: early weight streaming for small routed sets (MXFP4 / MXFP8 activations, at most 32
     local routes expected), turned on by the buffer's ``_debug_flags`` bit 3, and tail half units
     for up to 32 routes (A-MXFP4 / A-MXFP8 at H = 3072: the last round of L1 units, when at most
