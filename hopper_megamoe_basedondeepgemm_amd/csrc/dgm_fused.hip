@@ -541,8 +541,8 @@ DGM_DEV bool spin_until2(const int* p, int target, int limit, int* err, int* her
 // fragments (K-tile kt, column c, lane group g) are dealt out as f = (kt n + c) 4 + g to thread
 // f % 512: with one or two routes per expert, one or two waves load and store a slab and the rest
 // skip it. (Against fixed columns per lane, the empty ones stored as zeros by every wave: QoQ at 16
-// tokens 126.1 -> 122.1 us, A-MXFP8 at 8 tokens 75.3 -> 74.7, A-MXFP8 at 512 448 -> 446; NVFP4 at 64
-// tokens 345.0 -> 343.9; 2 to 13 VGPRs fewer.)
+// tokens 126.1 -> 122.1 us; A-MXFP8 at 8 and 512 tokens and NVFP4 at 64 less than 1 % faster, no more
+// than builds differ by their code layout; 2 to 13 VGPRs fewer.)
 template <int KT, int ACT, bool COHERENT, bool MIDL = COHERENT>
 struct SlabRegs {
   static constexpr int FR = (KT * 64 + FT - 1) / FT;
@@ -768,8 +768,8 @@ DGM_DEV long long wall_clock() { return (long long)__builtin_amdgcn_s_memrealtim
 // dispatch. It runs one phase per launch (L1, or L2 without the combine, which is a launch of its
 // own) and so has no wait on another workgroup: calls beyond the plain form's limits never needed
 // the whole grid resident, and two of them on two streams must not wait for each other's CUs.
-// E384 H3072 I1280, 512 tokens, whole call: A-MXFP8 442 us (259 L1, 151 L2 when first measured, at
-// 456; 1.71 + 0.89 GB read, 6.6 and 5.9 TB/s), one of eight ranks' experts, A-MXFP4, 101 us. The
+// E384 H3072 I1280, 512 tokens, whole call: A-MXFP8 448 us (259 L1, 151 L2 when first measured, at
+// 456; 1.71 + 0.89 GB read, 6.6 and 5.9 TB/s), one of eight ranks' experts, A-MXFP4, 103 us. The
 // kernels it replaced (a one-workgroup dispatch, L1 and L2 that load an item's weights before its
 // first op) took 1227 and 367 us, with the VALU router. Bound by the weight stream and, in L2, the items' fixed cost.
 // Measured and not taken: the whole layer in one launch (455 / 101 us, but with the waits), runs of

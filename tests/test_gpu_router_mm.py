@@ -1,5 +1,5 @@
 """The frontend's matrix-core router tiles (beyond 64 tokens, where they are enough) against its one-wave
-rows (below 64 tokens): fp32 logits, top-k keys and activation bytes bit for bit, with ragged token and expert
+rows (below 64 tokens), and beyond 64 tokens the rows of eight tokens where tiles are few: fp32 logits, top-k keys and activation bytes bit for bit, with ragged token and expert
 tiles, every hidden size, zero rows, subnormal and huge values, infinities and NaN; and the logits
 of the finite rows against the oracle's fixed order."""
 import numpy as np
@@ -14,7 +14,9 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("M,E,H,act", [(112, 384, 3072, "mxfp8"), (129, 48, 512, "mxfp4"), (143, 8, 1024, "qoq"),
                                        (160, 1000, 512, "nvfp4"), (200, 72, 2048, "fp8f128"), (131, 20, 4096, "mxfp8"),
-                                       (65, 200, 4096, "mxfp4"), (65, 8, 512, "mxfp8"), (111, 150, 3072, "fp8f128")])
+                                       (65, 200, 4096, "mxfp4"), (65, 8, 512, "mxfp8"), (111, 150, 3072, "fp8f128"),
+                                       # (few tiles: rows of eight tokens, the last ragged)
+                                       (70, 48, 2048, "mxfp4"), (101, 20, 3072, "mxfp8")])
 def test_router_tiles_equal_router_rows(M, E, H, act):
     need_gpu()
     import hopper_megamoe_basedondeepgemm_amd as dgm

@@ -114,3 +114,33 @@ def test_raw_weights_selected_by_the_layer_call(fmt, split, M, flags):
         assert torch.equal(u, v)
     if "forced" not in flags:
         assert torch.equal(out[1][3], logits.float().sort(dim=1, descending=True).values[:, :TOPK])
+
+
+@pytest.mark.parametrize("fmt,M", [("mxfp8", 20), ("fp8f128", 300)])
+def test_graph_replays(fmt, M):
+    """A captured split call replayed with other routings, eager calls and a one-launch call between the
+    replays: every replay gives the eager result bit for bit."""
+    need_gpu()
+    import hopper_megamoe_basedondeepgemm_amd as dgm
+    print(f"graph replays fmt={fmt} M={M}", flush=True)
+    l1, l2, buf = _filled(dgm, fmt, M)
+    weights = [buf.topk_weights.clone() * f for f in (1.0, 0.5, 2.0)]
+    refs = []
+    for w in weights:
+        buf.topk_weights.copy_(w)
+        refs.append(_call(dgm, l1, l2, buf, M))
+    y = torch.empty((M, H), dtype=torch.bfloat16, device="cuda")
+    stats = torch.zeros(E, dtype=torch.int32, device="cuda")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        dgm.mega._fused(y, l1, l2, buf, stats, 10.0, split=True)
+    for i in (0, 1, 2, 1):
+        buf.topk_weights.copy_(weights[i])
+        y.fill_(7.0)
+        stats.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.int16), refs[i][0]) and torch.equal(stats, refs[i][1]), i
+        for split in (True, False):
+            for u, v in zip(_call(dgm, l1, l2, buf, M, split), refs[i]):
+                assert torch.equal(u, v), i
